@@ -51,6 +51,16 @@ int tri_prepare_qk(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, cons
 int tri_pack_v(const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hk, int t, float* partial,
                float* vstat, void* v16p, void* v8p, void* v4p, int32_t* v8sum, void* stream);
 
+/* No counterpart in the reference: tri_prepare_qk, tri_pack_v and (exact not NULL)
+ * tri_pack_exact of one prompt in two launches (extension).  The arguments are
+ * theirs, with the same contracts; kpartial and vpartial are two scratch buffers
+ * (tri_pack_v may otherwise reuse tri_prepare_qk's). */
+int tri_prepare(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb, int64_t k_sh,
+                int64_t k_st, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hq, int hk, int t,
+                void* q8, float* qa, void* kp, float* ka, float* kpartial, float* kstat, void* q4, float* qa4,
+                void* k4p, float* ka4, void* k4x, float* vpartial, float* vstat, void* v16p, void* v8p, void* v4p,
+                int32_t* v8sum, const int32_t* exact, int nx, void* kx, void* vx, void* stream);
+
 /* Replaces attention (prefill_sm80.cu:510-543), band-table form only (the
  * reference's task-table form has no caller, prefill.py:103).
  * order int32 [n_order = hq*tiles]: workgroup -> qhead*tiles + qtile.

@@ -83,15 +83,12 @@ static int device_cus(int* cus) {
   return 0;
 }
 
-extern "C" {
-
-const char* tri_last_error(void) { return g_error.c_str(); }
-
-int tri_prepare_qk(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,
-                   int64_t k_sh, int64_t k_st, int batch, int hq, int hk, int t, void* q8, float* qa, void* kp,
-                   float* ka, float* partial, float* kstat, void* q4, float* qa4, void* k4p, float* ka4,
-                   void* k4x, void* stream) {
-  g_error.clear();
+// ---- prepare calls (tri_prepare_qk, tri_pack_v, tri_pack_exact, tri_prepare): argument checks of each part, and
+// the two launches that serve any combination of them
+static int prepare_qk_args(tri::PrepareArgs& a, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k,
+                           int64_t k_sb, int64_t k_sh, int64_t k_st, int batch, int hq, int hk, int t, void* q8,
+                           float* qa, void* kp, float* ka, float* partial, float* kstat, void* q4, float* qa4,
+                           void* k4p, float* ka4, void* k4x) {
   if (!q || !k || !q8 || !qa || !kp || !ka || !partial || !kstat) return fail("prepare_qk: null buffer");
   if (batch < 1 || hq < 1 || hk < 1 || t < 1) return fail("prepare_qk: empty shape");
   if (hq % hk != 0) return fail("prepare_qk: q heads (%d) not a multiple of kv heads (%d)", hq, hk);
@@ -103,42 +100,152 @@ int tri_prepare_qk(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, cons
   if (!aligned(kp, 16) || !aligned(q8, 16) || (int4 && (!aligned(k4p, 16) || !aligned(q4, 4))))
     return fail("prepare_qk: output buffers must be 16-byte aligned");
   if (k4x && (!int4 || !aligned(k4x, 16))) return fail("prepare_qk: expanded K4 records need the INT4 buffers, 16-byte aligned");
-  const int tiles = (t + tri::BN - 1) / tri::BN;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  tri::quantize_q_kernel<<<dim3((t + 31) / 32, hq, batch), 256, 0, s>>>(
-      static_cast<const uint16_t*>(q), q_sb, q_sh, q_st, hq, t, static_cast<int8_t*>(q8), qa,
-      static_cast<uint8_t*>(q4), qa4);
-  tri::partial_kernel<<<dim3(tri::STAT_BLOCKS, hk, batch), tri::D / 2, 0, s>>>(static_cast<const uint16_t*>(k), k_sb,
-                                                                          k_sh, k_st, hk, t, partial);
-  tri::finalize_kernel<<<dim3(hk, batch), tri::D, 0, s>>>(partial, kstat, hk, t, 0);
-  tri::quantize_k_kernel<<<dim3(tiles, hk, batch), 256, 0, s>>>(static_cast<const uint16_t*>(k), k_sb, k_sh, k_st,
-                                                                kstat, hk, t, static_cast<uint8_t*>(kp), ka,
-                                                                static_cast<uint8_t*>(k4p), ka4,
-                                                                static_cast<uint8_t*>(k4x));
-  return check_launch("prepare_qk");
+  a.q = static_cast<const uint16_t*>(q);
+  a.qsb = q_sb;
+  a.qsh = q_sh;
+  a.qst = q_st;
+  a.k = static_cast<const uint16_t*>(k);
+  a.ksb = k_sb;
+  a.ksh = k_sh;
+  a.kst = k_st;
+  a.batch = batch;
+  a.hq = hq;
+  a.hk = hk;
+  a.t = t;
+  a.q8 = static_cast<int8_t*>(q8);
+  a.qa = qa;
+  a.q4 = static_cast<uint8_t*>(q4);
+  a.qa4 = qa4;
+  a.k8 = static_cast<uint8_t*>(kp);
+  a.ka = ka;
+  a.k4 = static_cast<uint8_t*>(k4p);
+  a.ka4 = ka4;
+  a.k4x = static_cast<uint8_t*>(k4x);
+  a.kpart = partial;
+  a.kstat = kstat;
+  return 0;
 }
 
-int tri_pack_v(const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hk, int t, float* partial,
-               float* vstat, void* v16p, void* v8p, void* v4p, int32_t* v8sum, void* stream) {
-  g_error.clear();
+static int pack_v_args(tri::PrepareArgs& a, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hk,
+                       int t, float* partial, float* vstat, void* v16p, void* v8p, void* v4p, int32_t* v8sum) {
   if (!v || !partial || !vstat) return fail("pack_v: null buffer");
   if (batch < 1 || hk < 1 || t < 1) return fail("pack_v: empty shape");
   if (!aligned(v, 8) || (v_st | v_sh | v_sb) % 4 != 0) return fail("pack_v: V rows must be 8-byte aligned");
   if ((v16p && !aligned(v16p, 16)) || (v8p && !aligned(v8p, 16)) || (v4p && !aligned(v4p, 8)))
     return fail("pack_v: record buffers must be 16-byte aligned");
   if (v8sum && (!v8p || !aligned(v8sum, 16))) return fail("pack_v: V8 sums need the V8 records, 16-byte aligned");
+  a.v = static_cast<const uint16_t*>(v);
+  a.vsb = v_sb;
+  a.vsh = v_sh;
+  a.vst = v_st;
+  a.batch = batch;
+  a.hk = hk;
+  a.t = t;
+  a.vpart = partial;
+  a.vstat = vstat;
+  a.v_identity = v8p == nullptr && v4p == nullptr;
+  a.v16 = static_cast<uint8_t*>(v16p);
+  a.v8 = static_cast<uint8_t*>(v8p);
+  a.v4 = static_cast<uint8_t*>(v4p);
+  a.v8s = v8sum;
+  return 0;
+}
+
+static int pack_exact_args(tri::PrepareArgs& a, const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v,
+                           int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hq, int hk, int t,
+                           const int32_t* exact, int nx, void* kx, void* vx) {
   const int tiles = (t + tri::BN - 1) / tri::BN;
-  const bool identity = v8p == nullptr && v4p == nullptr;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!identity)
-    tri::partial_kernel<<<dim3(tri::STAT_BLOCKS, hk, batch), tri::D / 2, 0, s>>>(static_cast<const uint16_t*>(v), v_sb,
-                                                                            v_sh, v_st, hk, t, partial);
-  tri::finalize_kernel<<<dim3(hk, batch), tri::D, 0, s>>>(partial, vstat, hk, t, identity ? 1 : 0);
-  tri::pack_v_kernel<<<dim3(tiles, hk, batch), 256, 0, s>>>(static_cast<const uint16_t*>(v), v_sb, v_sh, v_st, vstat,
-                                                            hk, t, static_cast<uint8_t*>(v16p),
-                                                            static_cast<uint8_t*>(v8p), static_cast<uint8_t*>(v4p),
-                                                            v8sum);
-  return check_launch("pack_v");
+  if (!k || !v || !exact || !kx || !vx) return fail("pack_exact: null buffer");
+  if (batch < 1 || hq < 1 || hk < 1 || t < 1) return fail("pack_exact: empty shape");
+  if (tiles > tri::MAX_TILES) return fail("pack_exact: at most 131072 tokens");
+  if (hq % hk != 0) return fail("pack_exact: q heads not a multiple of kv heads");
+  if (nx < 1 || nx > hk) return fail("pack_exact: nx must be in [1, hk]");
+  if (!aligned(k, 16) || !aligned(v, 16) || (k_sb | k_sh | k_st | v_sb | v_sh | v_st) % 8 != 0)
+    return fail("pack_exact: K/V rows must be 16-byte aligned");
+  if (!aligned(kx, 16) || !aligned(vx, 16)) return fail("pack_exact: KX/VX records must be 16-byte aligned");
+  a.k = static_cast<const uint16_t*>(k);
+  a.ksb = k_sb;
+  a.ksh = k_sh;
+  a.kst = k_st;
+  a.v = static_cast<const uint16_t*>(v);
+  a.vsb = v_sb;
+  a.vsh = v_sh;
+  a.vst = v_st;
+  a.batch = batch;
+  a.hq = hq;
+  a.hk = hk;
+  a.t = t;
+  a.exact = exact;
+  a.nx = nx;
+  a.kx = static_cast<uint8_t*>(kx);
+  a.vx = static_cast<uint8_t*>(vx);
+  return 0;
+}
+
+// The launches of the parts that are present (k8, v16 / v8 / v4 with vstat, exact).
+static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) {
+  const int64_t tiles = (a.t + tri::BN - 1) / tri::BN, heads = (int64_t)a.hk * a.batch;
+  const bool has_k = a.k8 != nullptr, has_v = a.vstat != nullptr;
+  const int64_t stat = heads * (tri::STAT_BLOCKS / 4);
+  const int64_t qwgs = a.q8 ? (int64_t)((a.t + 31) / 32) * a.hq * a.batch : 0;
+  // Tiles per record workgroup: one while that gives at most RECORD_WGS workgroups per part (a short prompt
+  // then has a workgroup per tile), more beyond, so that the statistics each workgroup forms anew stay cheap
+  // beside its tiles.
+  a.per = (int)std::max<int64_t>(1, heads * tiles / tri::RECORD_WGS);
+  a.chunks = (int)((tiles + a.per - 1) / a.per);
+  const int64_t rec = heads * a.chunks, xwgs = a.exact ? heads * tiles : 0;
+  const int64_t g1 = (has_k ? stat : 0) + (has_v && !a.v_identity ? stat : 0) + qwgs;
+  const int64_t g2 = (has_k ? rec : 0) + (has_v ? rec : 0) + xwgs;
+  if (g1 > INT32_MAX || g2 > INT32_MAX) return fail("%s: too many rows", what);
+  a.kstat_wgs = has_k ? (int)stat : 0;
+  a.vstat_wgs = has_v && !a.v_identity ? (int)stat : 0;
+  a.krec_wgs = has_k ? (int)rec : 0;
+  a.vrec_wgs = has_v ? (int)rec : 0;
+  if (g1 > 0) tri::prepare_stats_kernel<<<dim3((unsigned)g1), 256, 0, s>>>(a);
+  tri::prepare_records_kernel<<<dim3((unsigned)g2), 256, 0, s>>>(a);
+  return check_launch(what);
+}
+
+extern "C" {
+
+const char* tri_last_error(void) { return g_error.c_str(); }
+
+int tri_prepare_qk(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,
+                   int64_t k_sh, int64_t k_st, int batch, int hq, int hk, int t, void* q8, float* qa, void* kp,
+                   float* ka, float* partial, float* kstat, void* q4, float* qa4, void* k4p, float* ka4,
+                   void* k4x, void* stream) {
+  g_error.clear();
+  tri::PrepareArgs a = {};
+  if (prepare_qk_args(a, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, batch, hq, hk, t, q8, qa, kp, ka, partial, kstat, q4,
+                      qa4, k4p, ka4, k4x) != 0)
+    return 1;
+  return launch_prepare(a, static_cast<hipStream_t>(stream), "prepare_qk");
+}
+
+int tri_pack_v(const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hk, int t, float* partial,
+               float* vstat, void* v16p, void* v8p, void* v4p, int32_t* v8sum, void* stream) {
+  g_error.clear();
+  tri::PrepareArgs a = {};
+  a.hq = hk;
+  if (pack_v_args(a, v, v_sb, v_sh, v_st, batch, hk, t, partial, vstat, v16p, v8p, v4p, v8sum) != 0) return 1;
+  return launch_prepare(a, static_cast<hipStream_t>(stream), "pack_v");
+}
+
+int tri_prepare(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb, int64_t k_sh,
+                int64_t k_st, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batch, int hq, int hk, int t,
+                void* q8, float* qa, void* kp, float* ka, float* kpartial, float* kstat, void* q4, float* qa4,
+                void* k4p, float* ka4, void* k4x, float* vpartial, float* vstat, void* v16p, void* v8p, void* v4p,
+                int32_t* v8sum, const int32_t* exact, int nx, void* kx, void* vx, void* stream) {
+  g_error.clear();
+  tri::PrepareArgs a = {};
+  if (prepare_qk_args(a, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, batch, hq, hk, t, q8, qa, kp, ka, kpartial, kstat, q4,
+                      qa4, k4p, ka4, k4x) != 0 ||
+      pack_v_args(a, v, v_sb, v_sh, v_st, batch, hk, t, vpartial, vstat, v16p, v8p, v4p, v8sum) != 0)
+    return 1;
+  if (exact != nullptr &&
+      pack_exact_args(a, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st, batch, hq, hk, t, exact, nx, kx, vx) != 0)
+    return 1;
+  return launch_prepare(a, static_cast<hipStream_t>(stream), "prepare");
 }
 
 int tri_attention(const int32_t* order, int n_order, const int32_t* bands, int batch, int hq, int hk, int t,
@@ -231,33 +338,9 @@ int tri_pack_exact(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, cons
                    int64_t v_sh, int64_t v_st, int batch, int hq, int hk, int t, const int32_t* exact, int nx,
                    void* kx, void* vx, void* stream) {
   g_error.clear();
-  const int tiles = (t + tri::BN - 1) / tri::BN;
-  if (!k || !v || !exact || !kx || !vx) return fail("pack_exact: null buffer");
-  if (batch < 1 || hq < 1 || hk < 1 || t < 1) return fail("pack_exact: empty shape");
-  if (tiles > tri::MAX_TILES) return fail("pack_exact: at most 131072 tokens");
-  if (hq % hk != 0) return fail("pack_exact: q heads not a multiple of kv heads");
-  if (nx < 1 || nx > hk) return fail("pack_exact: nx must be in [1, hk]");
-  if (!aligned(k, 16) || !aligned(v, 16) || (k_sb | k_sh | k_st | v_sb | v_sh | v_st) % 8 != 0)
-    return fail("pack_exact: K/V rows must be 16-byte aligned");
-  if (!aligned(kx, 16) || !aligned(vx, 16)) return fail("pack_exact: KX/VX records must be 16-byte aligned");
-  tri::ExactPackArgs a;
-  a.k = static_cast<const uint16_t*>(k);
-  a.v = static_cast<const uint16_t*>(v);
-  a.ksb = k_sb;
-  a.ksh = k_sh;
-  a.kst = k_st;
-  a.vsb = v_sb;
-  a.vsh = v_sh;
-  a.vst = v_st;
-  a.exact = exact;
-  a.kx = static_cast<uint8_t*>(kx);
-  a.vx = static_cast<uint8_t*>(vx);
-  a.hq = hq;
-  a.hk = hk;
-  a.t = t;
-  a.nx = nx;
-  tri::pack_exact_kernel<<<dim3(tiles, hk, batch), 256, 0, static_cast<hipStream_t>(stream)>>>(a);
-  return check_launch("pack_exact");
+  tri::PrepareArgs a = {};
+  if (pack_exact_args(a, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st, batch, hq, hk, t, exact, nx, kx, vx) != 0) return 1;
+  return launch_prepare(a, static_cast<hipStream_t>(stream), "pack_exact");
 }
 
 static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8c, const void* k4c, const float* ka,

@@ -455,72 +455,6 @@ __device__ __forceinline__ void prefill_exact(const PrefillArgs& a, int b, int q
     }
 }
 
-// Packs the K and V of every exact KV head into KX / VX records (one workgroup
-// per (tile, KV head, sequence); other heads return at once).  Keys at or past
-// t are zero.  Per 64-key tile, 16 KiB each, 32-key half kb at byte kb*8192:
-//   KX fragment F = ks (16-feature step), lane L 16 bytes = bf16 K[key kb*32 + L%32]
-//      [features ks*16 + 8*(L/32) .. +7]      (A operand of S^T = K Q^T)
-//   VX fragment F = cb*2 + kh, lane L element e = bf16 V[key kb*32 + 16*kh + 8*(e/4)
-//      + 4*(L/32) + e%4][channel cb*32 + L%32] (A operand of O^T = V^T P^T)
-struct ExactPackArgs {
-  const uint16_t* k;
-  const uint16_t* v;
-  int64_t ksb, ksh, kst, vsb, vsh, vst;
-  const int32_t* exact;  // [hq]: 1 + record slot of the q-head's KV head, 0 if quantized
-  uint8_t* kx;
-  uint8_t* vx;
-  int hq, hk, t, nx;
-};
-
-// One tile of pack_exact: keys r < rows of ksrc / vsrc (row strides kst / vst) into the KX and VX
-// records kd / vd; vt is the workgroup's LDS staging of V.  256 threads.
-constexpr int EXACT_VP = D + 8;  // padded LDS row of the V staging (bf16 elements)
-__device__ __forceinline__ void pack_exact_tile(const uint16_t* ksrc, int64_t kst, const uint16_t* vsrc, int64_t vst,
-                                                int rows, uint8_t* kd, uint8_t* vd, uint16_t* vt) {
-  const int tid = threadIdx.x;
-  // K: 1024 16-byte pieces in source order (key, 8-feature piece)
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = tid + 256 * i, key = c >> 4, f0 = (c & 15) * 8;
-    uint4 w = make_uint4(0, 0, 0, 0), u = w;
-    if (key < rows) {
-      w = *reinterpret_cast<const uint4*>(ksrc + (int64_t)key * kst + f0);
-      u = *reinterpret_cast<const uint4*>(vsrc + (int64_t)key * vst + f0);
-    }
-    const int kb = key >> 5, lk = key & 31, ks = f0 >> 4, h = (f0 >> 3) & 1;
-    *reinterpret_cast<uint4*>(kd + kb * (KX_BYTES / 2) + ks * 1024 + (h * 32 + lk) * 16) = w;
-    *reinterpret_cast<uint4*>(vt + key * EXACT_VP + f0) = u;
-  }
-  __syncthreads();
-  // V: 1024 output pieces in destination order
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = tid + 256 * i, F = c >> 6, L = c & 63;  // F = kb*8 + cb*2 + kh
-    const int kb = F >> 3, cb = (F >> 1) & 3, khalf = F & 1, ch = cb * 32 + (L & 31), h = L >> 5;
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e0 = 2 * j, e1 = 2 * j + 1;
-      const int k0 = kb * 32 + 16 * khalf + 8 * (e0 >> 2) + 4 * h + (e0 & 3);
-      const int k1 = kb * 32 + 16 * khalf + 8 * (e1 >> 2) + 4 * h + (e1 & 3);
-      w[j] = (uint32_t)vt[k0 * EXACT_VP + ch] | ((uint32_t)vt[k1 * EXACT_VP + ch] << 16);
-    }
-    *reinterpret_cast<uint4*>(vd + c * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
-__global__ __launch_bounds__(256) void pack_exact_kernel(ExactPackArgs a) {
-  const int tile = blockIdx.x, kh = blockIdx.y, b = blockIdx.z;
-  const int slot = a.exact[kh * (a.hq / a.hk)] - 1;
-  if (slot < 0) return;
-  const int tiles = gridDim.x;
-  const int64_t rec = ((int64_t)b * a.nx + slot) * tiles + tile;
-  __shared__ __align__(16) uint16_t vt[BN * EXACT_VP];
-  pack_exact_tile(a.k + b * a.ksb + kh * a.ksh + (int64_t)tile * BN * a.kst, a.kst,
-                  a.v + b * a.vsb + kh * a.vsh + (int64_t)tile * BN * a.vst, a.vst, a.t - tile * BN,
-                  a.kx + rec * KX_BYTES, a.vx + rec * KX_BYTES, vt);
-}
-
 template <int V>
 struct Tag {
   static constexpr int value = V;

@@ -8,16 +8,46 @@
 
 namespace tri {
 
-// One 128-feature row per 8 lanes (16 features per lane, rotated with DPP lane
-// moves by rotate128_x16), 32 rows per 256-thread block.
-// common_device.cuh:1-28 (quantize_q_kernel).
-__global__ __launch_bounds__(256) void quantize_q_kernel(const uint16_t* __restrict__ q, int64_t sb, int64_t sh,
-                                                         int64_t st, int hq, int t, int8_t* __restrict__ q8,
-                                                         float* __restrict__ qa, uint8_t* __restrict__ q4,
-                                                         float* __restrict__ qa4) {
-  const int sub = threadIdx.x & 7, row = blockIdx.x * 32 + (threadIdx.x >> 3), h = blockIdx.y, b = blockIdx.z;
-  if (row >= t) return;  // whole 8-lane groups leave together
-  const uint16_t* src = q + b * sb + h * sh + (int64_t)row * st + sub * 16;
+// Record workgroups per part (K, V) up to which each takes a single tile.  Fewer workgroups form the
+// statistics less often, more have more loads in flight (prepare_records_kernel at 256 / 512 / 1024 / 2048:
+// 4 x 8192 tokens, 4 KV heads, 46 / 41 / 46 / 52 us; 30,001 tokens, 8 KV heads, 76 / 72 / 66 / 80 us).
+constexpr int RECORD_WGS = 512;
+
+// Arguments of one prepare call.  Parts that a call leaves out have a null source: q (the Q codes), k (K
+// statistics and records), v (V records; its statistics too unless v_identity), exact (KX / VX records).
+struct PrepareArgs {
+  const uint16_t *q, *k, *v;  // bf16 [B][H][T][128], strides in elements
+  int64_t qsb, qsh, qst, ksb, ksh, kst, vsb, vsh, vst;
+  int batch, hq, hk, t;
+  int8_t* q8;
+  float* qa;
+  uint8_t* q4;  // (q4, qa4, k4, ka4 null together)
+  float* qa4;
+  uint8_t* k8;
+  float* ka;
+  uint8_t* k4;
+  float* ka4;
+  uint8_t* k4x;  // may be null
+  float *kpart, *vpart;  // [B][Hk][64][3][128] block partials
+  float *kstat, *vstat;  // [B][Hk][3][128] mean, scale, 1 / scale
+  int v_identity;        // V' = V: no V8 or V4 records, statistics (0, 1, 1)
+  uint8_t *v16, *v8, *v4;  // may be null
+  int32_t* v8s;            // may be null
+  const int32_t* exact;    // [hq]: 1 + record slot of the q-head's KV head, 0 if quantized
+  int nx;
+  uint8_t *kx, *vx;
+  // workgroups per part and tiles per record workgroup (set by the host)
+  int kstat_wgs, vstat_wgs, krec_wgs, vrec_wgs, per, chunks;
+};
+
+// Q codes: one 128-feature row per 8 lanes (16 features per lane, rotated with DPP lane moves by
+// rotate128_x16), 32 rows per 256-thread workgroup.  common_device.cuh:1-28 (quantize_q_kernel).
+__device__ __forceinline__ void quantize_q_rows(const PrepareArgs& a, int wg) {
+  const int blocks = (a.t + 31) / 32;
+  const int sub = threadIdx.x & 7, row = (wg % blocks) * 32 + (threadIdx.x >> 3);
+  const int h = (wg / blocks) % a.hq, b = wg / (blocks * a.hq);
+  if (row >= a.t) return;  // whole 8-lane groups leave together
+  const uint16_t* src = a.q + b * a.qsb + h * a.qsh + (int64_t)row * a.qst + sub * 16;
   float x[16];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -32,7 +62,7 @@ __global__ __launch_bounds__(256) void quantize_q_kernel(const uint16_t* __restr
 #pragma unroll
   for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(x[i]));
   m = lanes8_max(m);
-  const int64_t r = ((int64_t)b * hq + h) * t + row;
+  const int64_t r = ((int64_t)b * a.hq + h) * a.t + row;
   const float inv = m > 0.f ? 127.f / m : 0.f;
   uint32_t w[4];
 #pragma unroll
@@ -41,38 +71,38 @@ __global__ __launch_bounds__(256) void quantize_q_kernel(const uint16_t* __restr
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[k] |= ((uint32_t)(int)__builtin_rintf(x[4 * k + i] * inv) & 0xffu) << (8 * i);
   }
-  *reinterpret_cast<uint4*>(q8 + r * D + sub * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  if (sub == 0) qa[r] = m / 127.f;
-  if (q4 != nullptr) {
+  *reinterpret_cast<uint4*>(a.q8 + r * D + sub * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  if (sub == 0) a.qa[r] = m / 127.f;
+  if (a.q4 != nullptr) {
     const float inv4 = m > 0.f ? 7.f / m : 0.f;
     uint32_t nib[2] = {0u, 0u};
 #pragma unroll
     for (int i = 0; i < 16; ++i) nib[i >> 3] |= ((uint32_t)(int)__builtin_rintf(x[i] * inv4) & 0xfu) << (4 * (i & 7));
-    uint32_t* dst = reinterpret_cast<uint32_t*>(q4 + r * (D / 2) + sub * 8);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(a.q4 + r * (D / 2) + sub * 8);
     dst[0] = nib[0];
     dst[1] = nib[1];
-    if (sub == 0) qa4[r] = m / 7.f;
+    if (sub == 0) a.qa4[r] = m / 7.f;
   }
 }
 
 // Per channel: sequential sum/max/min over tokens t = blk, blk+64, ...
-// common_device.cuh:32-42 (partial_kernel).  partial [B][H][64][3][128].
-// Lane i takes channels 2i and 2i + 1 (one 4-byte load per token; rows are 8-byte aligned) and
-// issues the loads of STAT_DEPTH tokens before it adds them, in token order, so each channel's
-// sum is formed in the reference's order while 32 loads per lane are in flight (C2's K: 14 us
-// against 22 us with 2-byte loads four deep; 64 deep, or 8 channels per lane with two rows per
-// load, measured no faster).
-constexpr int STAT_DEPTH = 32;
-__global__ __launch_bounds__(64) void partial_kernel(const uint16_t* __restrict__ x, int64_t sb, int64_t sh,
-                                                     int64_t st, int h, int t, float* __restrict__ partial) {
-  const int blk = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, c = 2 * threadIdx.x;
-  const uint16_t* base = x + b * sb + hd * sh + c;
+// common_device.cuh:32-42 (partial_kernel).  One wave per (blk, head): lane i takes channels 2i and
+// 2i + 1 (one 4-byte load per token; rows are 8-byte aligned).  Each channel's sum is formed in the
+// reference's token order, so the chain is serial; the loads are not: the next STAT_DEPTH tokens load
+// while the current ones are added.
+constexpr int STAT_DEPTH = 16;
+__device__ __forceinline__ void stat_block(const uint16_t* __restrict__ src, int64_t st, int t, int blk,
+                                           float* __restrict__ partial) {
+  const int c = 2 * (threadIdx.x & 63);
   float sum0 = 0.f, sum1 = 0.f, hi0 = -3.402823466e38f, hi1 = hi0, lo0 = 3.402823466e38f, lo1 = lo0;
-  for (int tk = blk; tk < t; tk += STAT_DEPTH * STAT_BLOCKS) {
-    uint32_t w[STAT_DEPTH];
+  uint32_t cur[STAT_DEPTH], nxt[STAT_DEPTH];
+  auto load = [&](uint32_t (&w)[STAT_DEPTH], int tk) {
 #pragma unroll
     for (int j = 0; j < STAT_DEPTH; ++j)
-      if (tk + j * STAT_BLOCKS < t) w[j] = *reinterpret_cast<const uint32_t*>(base + (int64_t)(tk + j * STAT_BLOCKS) * st);
+      if (tk + j * STAT_BLOCKS < t)
+        w[j] = *reinterpret_cast<const uint32_t*>(src + (int64_t)(tk + j * STAT_BLOCKS) * st + c);
+  };
+  auto add = [&](const uint32_t (&w)[STAT_DEPTH], int tk) {
 #pragma unroll
     for (int j = 0; j < STAT_DEPTH; ++j)
       if (tk + j * STAT_BLOCKS < t) {
@@ -84,40 +114,117 @@ __global__ __launch_bounds__(64) void partial_kernel(const uint16_t* __restrict_
         lo0 = fminf(lo0, v0);
         lo1 = fminf(lo1, v1);
       }
+  };
+  constexpr int STEP = STAT_DEPTH * STAT_BLOCKS;
+  load(cur, blk);
+  for (int tk = blk; tk < t; tk += 2 * STEP) {
+    load(nxt, tk + STEP);
+    add(cur, tk);
+    load(cur, tk + 2 * STEP);
+    add(nxt, tk + STEP);
   }
-  float* o = partial + ((((int64_t)b * h + hd) * STAT_BLOCKS + blk) * 3) * D + c;
+  float* o = partial + (int64_t)blk * 3 * D + c;
   *reinterpret_cast<float2*>(o) = make_float2(sum0, sum1);
   *reinterpret_cast<float2*>(o + D) = make_float2(hi0, hi1);
   *reinterpret_cast<float2*>(o + 2 * D) = make_float2(lo0, lo1);
 }
 
-// mean = (sum of block sums in block order) / T, scale = range/127 (1 if 0),
-// inv = 1/scale; identity mode writes (0, 1, 1).  common_device.cuh:44-56.
-__global__ __launch_bounds__(128) void finalize_kernel(const float* __restrict__ partial, float* __restrict__ stat,
-                                                       int h, int t, int identity) {
-  const int hd = blockIdx.x, b = blockIdx.y, c = threadIdx.x;
-  const int64_t hb = (int64_t)b * h + hd;
-  float mean = 0.f, scale = 1.f;
-  if (!identity) {
-    const float* in = partial + hb * STAT_BLOCKS * 3 * D + c;
-    float sum = 0.f, hi = -3.402823466e38f, lo = 3.402823466e38f;
-    // (unrolled: the 192 loads issue together, and the sum still runs in block order)
+// First launch of a prepare call: the K and V statistics' block partials and the Q codes, which depend on
+// nothing but the inputs.  The statistics are latency-bound (64 serial sums per head and channel pair, one
+// wave each) and come first in the grid; the Q codes are HBM-bound and fill the rest of the chip meanwhile
+// (64 VGPRs at most, so that eight waves per SIMD keep their loads in flight).  Against a launch each
+// (Q codes, K partials, V partials): 4 x 8192 tokens, Hq 28 / Hk 4, 111 -> 105 us (4.6 TB/s, a plain copy
+// reaches 4.85); 30,001 tokens, Hq 32 / Hk 8, 163 -> 109 us; 1,024 tokens, Hq 24 / Hk 8, 14 -> 7.8 us.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void prepare_stats_kernel(PrepareArgs a) {
+  int wg = blockIdx.x;
+  if (wg < a.kstat_wgs + a.vstat_wgs) {
+    const bool isv = wg >= a.kstat_wgs;
+    if (isv) wg -= a.kstat_wgs;
+    const int hb = wg / (STAT_BLOCKS / 4), blk = (wg % (STAT_BLOCKS / 4)) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int hd = hb % a.hk, b = hb / a.hk;
+    const uint16_t* src = isv ? a.v + b * a.vsb + hd * a.vsh : a.k + b * a.ksb + hd * a.ksh;
+    stat_block(src, isv ? a.vst : a.kst, a.t, blk, (isv ? a.vpart : a.kpart) + (int64_t)hb * STAT_BLOCKS * 3 * D);
+    return;
+  }
+  quantize_q_rows(a, wg - a.kstat_wgs - a.vstat_wgs);
+}
+
+// Statistics of one head from its block partials: mean = (sum of block sums in block order) / T, scale =
+// range/127 (1 if 0), inv = 1/scale.  common_device.cuh:44-56 (finalize_kernel).  Every record workgroup
+// forms them again (96 KiB of partials, L2-resident) instead of waiting for a launch that does nothing
+// else.  256 threads: one half adds the channel's block sums, the other takes its extremes; mean and
+// inv (LDS, 128 each) are complete after the call's barrier.  stat (when not null) receives all three.
+// `range`: whether scale and inv are needed (a K record needs the mean alone).
+__device__ __forceinline__ void head_stats(const float* __restrict__ partial, int t, bool range, float* mean_lds,
+                                           float* inv_lds, float* hi_lds, float* lo_lds, float* __restrict__ stat) {
+  const int c = threadIdx.x & (D - 1);
+  const float* in = partial + c;
+  float sum = 0.f;
+  if (threadIdx.x < D) {
+    // (unrolled: the 64 loads issue together, and the sum still runs in block order)
 #pragma unroll
+    for (int blk = 0; blk < STAT_BLOCKS; ++blk) sum += in[blk * 3 * D];
+  } else if (range) {
+    float hi = -3.402823466e38f, lo = 3.402823466e38f;
+#pragma unroll 32
     for (int blk = 0; blk < STAT_BLOCKS; ++blk) {
-      sum += in[blk * 3 * D];
       hi = fmaxf(hi, in[blk * 3 * D + D]);
       lo = fminf(lo, in[blk * 3 * D + 2 * D]);
     }
-    mean = sum / (float)t;
-    const float range = fmaxf(hi - mean, mean - lo);
-    scale = range > 0.f ? range / 127.f : 1.f;
+    hi_lds[c] = hi;
+    lo_lds[c] = lo;
   }
-  stat[hb * 3 * D + c] = mean;
-  stat[hb * 3 * D + D + c] = scale;
-  stat[hb * 3 * D + 2 * D + c] = 1.f / scale;
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const float mean = sum / (float)t;
+    mean_lds[c] = mean;
+    if (range) {
+      const float r = fmaxf(hi_lds[c] - mean, mean - lo_lds[c]);
+      const float scale = r > 0.f ? r / 127.f : 1.f;
+      inv_lds[c] = 1.f / scale;
+      if (stat != nullptr) {
+        stat[c] = mean;
+        stat[D + c] = scale;
+        stat[2 * D + c] = 1.f / scale;
+      }
+    }
+  }
+  __syncthreads();
 }
 
-// y = R(k - mean) of one 64-key tile: rows src + r * st for r < rows (zeros past); the INT8 record rec8
+// A 64-key tile's bf16 rows src + r * st (r < rows), loaded ahead of their use: quantize_k_tile's key
+// layout (wave w rows 16w..16w+15 in two passes of 8 keys, 16 features per lane) and pack_v_tile's (four
+// channels per thread, 8 rows apart).
+struct KRaw {
+  uint2 w[2][4];
+};
+struct VRaw {
+  uint2 w[8];
+};
+__device__ __forceinline__ void load_k_tile(KRaw& raw, const uint16_t* __restrict__ src, int64_t st, int rows) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int r = wave * 16 + it * 8 + (lane >> 3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw.w[it][i] = make_uint2(0u, 0u);
+    if (r < rows) {
+      const uint16_t* row = src + (int64_t)r * st + (lane & 7) * 16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) raw.w[it][i] = *reinterpret_cast<const uint2*>(row + 4 * i);
+    }
+  }
+}
+__device__ __forceinline__ void load_v_tile(VRaw& raw, const uint16_t* __restrict__ src, int64_t st, int rows) {
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    const int r = n * 8 + (threadIdx.x >> 5), c0 = (threadIdx.x & 31) * 4;
+    raw.w[n] = make_uint2(0u, 0u);
+    if (r < rows) raw.w[n] = *reinterpret_cast<const uint2*>(src + (int64_t)r * st + c0);
+  }
+}
+
+// y = R(k - mean) of one 64-key tile: the rows of raw below `rows` (zeros past); the INT8 record rec8
 // with its four group scales ka, and the INT4 record rec4 with ka4 (either pair may be null).  Wave w
 // owns the 16-key group w, one key per 8 lanes (16 features per lane, DPP rotation), two passes of 8
 // keys; c8 / c4 are the workgroup's LDS staging.  256 threads.
@@ -125,7 +232,7 @@ __global__ __launch_bounds__(128) void finalize_kernel(const float* __restrict__
 // Extension: rec4x (with rec4; may be null) receives the INT4 codes once more, expanded to one byte of
 // 16 * code each in the INT8 record's layout (8 KiB): the bytes the prefill kernel would otherwise expand
 // from rec4 in every tile it reads.
-__device__ __forceinline__ void quantize_k_tile(const uint16_t* __restrict__ src, int64_t st, int rows,
+__device__ __forceinline__ void quantize_k_tile(const KRaw& in, int rows,
                                                 const float* __restrict__ mean, uint8_t* __restrict__ rec8,
                                                 float* __restrict__ ka, uint8_t* __restrict__ rec4,
                                                 float* __restrict__ ka4, uint8_t (*c8)[D], uint8_t (*c4)[D],
@@ -143,10 +250,9 @@ __device__ __forceinline__ void quantize_k_tile(const uint16_t* __restrict__ src
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = 0.f;
     if (r < rows) {
-      const uint16_t* row = src + (int64_t)r * st + sub * 16;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(row + 4 * i);
+        const uint2 raw = in.w[it][i];
         x[4 * i] = bf16f(raw.x & 0xffffu) - mc[4 * i];
         x[4 * i + 1] = bf16f(raw.x >> 16) - mc[4 * i + 1];
         x[4 * i + 2] = bf16f(raw.y & 0xffffu) - mc[4 * i + 2];
@@ -207,38 +313,24 @@ __device__ __forceinline__ void quantize_k_tile(const uint16_t* __restrict__ src
   }
 }
 
-// quantize_k_tile for every (tile, KV head, sequence): K [B][Hk][T][128] into [B][Hk][tiles] records.
-__global__ __launch_bounds__(256) void quantize_k_kernel(const uint16_t* __restrict__ k, int64_t sb, int64_t sh,
-                                                         int64_t st, const float* __restrict__ kstat, int hk, int t,
-                                                         uint8_t* __restrict__ k8, float* __restrict__ ka,
-                                                         uint8_t* __restrict__ k4, float* __restrict__ ka4,
-                                                         uint8_t* __restrict__ k4x) {
-  __shared__ __align__(16) uint8_t c8[BN][D];
-  __shared__ __align__(16) uint8_t c4[BN][D];
-  const int tile = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, tiles = (t + BN - 1) / BN;
-  const int64_t hb = (int64_t)b * hk + hd, rec = hb * tiles + tile;
-  quantize_k_tile(k + b * sb + hd * sh + (int64_t)tile * BN * st, st, t - tile * BN, kstat + hb * 3 * D,
-                  k8 + rec * K8_BYTES, ka + rec * 4, k4 != nullptr ? k4 + rec * K4_BYTES : nullptr,
-                  k4 != nullptr ? ka4 + rec * 4 : nullptr, c8, c4, k4x != nullptr ? k4x + rec * K8_BYTES : nullptr);
-}
-
-// v' = (v - mean) * inv of one 64-key tile (rows src + r * st for r < rows, zeros past) into the V16
+// v' = (v - mean) * inv of one 64-key tile (the rows of raw below `rows`, zeros past) into the V16
 // (fp16), V8 and V4 records (any may be null); vn is the workgroup's LDS staging.  256 threads.
 // common_device.cuh:132-172 (vnorm, pack_v_kernel).
 // Extension: v8s (with v8; may be null) receives -127 times each channel's sum of the tile's 64 V8 codes
 // (int32 [128], channel order), the value the prefill's P V product starts from (vsum: LDS of 128 ints).
-__device__ __forceinline__ void pack_v_tile(const uint16_t* __restrict__ src, int64_t st, int rows,
+__device__ __forceinline__ void pack_v_tile(const VRaw& in, int rows,
                                             const float* __restrict__ mean, const float* __restrict__ inv,
                                             uint8_t* __restrict__ v16, uint8_t* __restrict__ v8,
                                             uint8_t* __restrict__ v4, float (*vn)[D + 1],
                                             int32_t* __restrict__ v8s = nullptr, int* vsum = nullptr) {
   const int tid = threadIdx.x;
   if (v8s != nullptr && tid < D) vsum[tid] = 0;
-  for (int i = tid; i < BN * D / 4; i += 256) {
-    const int r = i / (D / 4), c0 = (i % (D / 4)) * 4;
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    const int r = n * 8 + (tid >> 5), c0 = (tid & 31) * 4;
     float x[4] = {0.f, 0.f, 0.f, 0.f};
     if (r < rows) {
-      const uint2 raw = *reinterpret_cast<const uint2*>(src + (int64_t)r * st + c0);
+      const uint2 raw = in.w[n];
       x[0] = (bf16f(raw.x & 0xffffu) - mean[c0]) * inv[c0];
       x[1] = (bf16f(raw.x >> 16) - mean[c0 + 1]) * inv[c0 + 1];
       x[2] = (bf16f(raw.y & 0xffffu) - mean[c0 + 2]) * inv[c0 + 2];
@@ -291,19 +383,125 @@ __device__ __forceinline__ void pack_v_tile(const uint16_t* __restrict__ src, in
   }
 }
 
-// pack_v_tile for every (tile, KV head, sequence): V [B][Hk][T][128] into [B][Hk][tiles] records.
-__global__ __launch_bounds__(256) void pack_v_kernel(const uint16_t* __restrict__ v, int64_t sb, int64_t sh,
-                                                     int64_t st, const float* __restrict__ vstat, int hk, int t,
-                                                     uint8_t* __restrict__ v16, uint8_t* __restrict__ v8,
-                                                     uint8_t* __restrict__ v4, int32_t* __restrict__ v8s) {
-  __shared__ float vn[BN][D + 1];
+// The KX / VX records of the exact KV heads.  Keys at or past t are zero.  Per 64-key tile, 16 KiB each, 32-key half kb at byte kb*8192:
+//   KX fragment F = ks (16-feature step), lane L 16 bytes = bf16 K[key kb*32 + L%32]
+//      [features ks*16 + 8*(L/32) .. +7]      (A operand of S^T = K Q^T)
+//   VX fragment F = cb*2 + kh, lane L element e = bf16 V[key kb*32 + 16*kh + 8*(e/4)
+//      + 4*(L/32) + e%4][channel cb*32 + L%32] (A operand of O^T = V^T P^T)
+// One tile: keys r < rows of ksrc / vsrc (row strides kst / vst) into the KX and VX
+// records kd / vd; vt is the workgroup's LDS staging of V.  256 threads.
+constexpr int EXACT_VP = D + 8;  // padded LDS row of the V staging (bf16 elements)
+__device__ __forceinline__ void pack_exact_tile(const uint16_t* ksrc, int64_t kst, const uint16_t* vsrc, int64_t vst,
+                                                int rows, uint8_t* kd, uint8_t* vd, uint16_t* vt) {
+  const int tid = threadIdx.x;
+  // K: 1024 16-byte pieces in source order (key, 8-feature piece)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = tid + 256 * i, key = c >> 4, f0 = (c & 15) * 8;
+    uint4 w = make_uint4(0, 0, 0, 0), u = w;
+    if (key < rows) {
+      w = *reinterpret_cast<const uint4*>(ksrc + (int64_t)key * kst + f0);
+      u = *reinterpret_cast<const uint4*>(vsrc + (int64_t)key * vst + f0);
+    }
+    const int kb = key >> 5, lk = key & 31, ks = f0 >> 4, h = (f0 >> 3) & 1;
+    *reinterpret_cast<uint4*>(kd + kb * (KX_BYTES / 2) + ks * 1024 + (h * 32 + lk) * 16) = w;
+    *reinterpret_cast<uint4*>(vt + key * EXACT_VP + f0) = u;
+  }
+  __syncthreads();
+  // V: 1024 output pieces in destination order
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = tid + 256 * i, F = c >> 6, L = c & 63;  // F = kb*8 + cb*2 + kh
+    const int kb = F >> 3, cb = (F >> 1) & 3, khalf = F & 1, ch = cb * 32 + (L & 31), h = L >> 5;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int e0 = 2 * j, e1 = 2 * j + 1;
+      const int k0 = kb * 32 + 16 * khalf + 8 * (e0 >> 2) + 4 * h + (e0 & 3);
+      const int k1 = kb * 32 + 16 * khalf + 8 * (e1 >> 2) + 4 * h + (e1 & 3);
+      w[j] = (uint32_t)vt[k0 * EXACT_VP + ch] | ((uint32_t)vt[k1 * EXACT_VP + ch] << 16);
+    }
+    *reinterpret_cast<uint4*>(vd + c * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// Second launch of a prepare call: the K records, the V records and the exact heads' KX / VX records.  A K
+// or V workgroup forms its head's statistics from the block partials, then takes a.per consecutive tiles;
+// the first one of a head writes the statistics out.  HBM-bound for long prompts, latency-bound for short
+// ones: a tile's rows are loaded before the statistics, and the next tile's while one is worked on.
+// Against launches of their own for each head's statistics (K, V), the K, V and KX / VX records: 4 x 8192
+// tokens, 4 KV heads (one exact), 54 -> 41 us; 1,024 tokens, 8 KV heads, 20 -> 9 us.
+__global__ __launch_bounds__(256) void prepare_records_kernel(PrepareArgs a) {
+  // one staging buffer for the three parts: V' of a tile (fp32), K codes (one byte each, INT8 and INT4), or
+  // the exact heads' bf16 V
+  __shared__ __align__(16) float stage[BN][D + 1];
+  __shared__ float mean[D], inv[D], hi[D], lo[D];
   __shared__ int vsum[D];
-  const int tile = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, tiles = (t + BN - 1) / BN;
-  const int64_t hb = (int64_t)b * hk + hd, rec = hb * tiles + tile;
-  const float* mean = vstat + hb * 3 * D;
-  pack_v_tile(v + b * sb + hd * sh + (int64_t)tile * BN * st, st, t - tile * BN, mean, mean + 2 * D,
-              v16 != nullptr ? v16 + rec * V16_BYTES : nullptr, v8 != nullptr ? v8 + rec * V8_BYTES : nullptr,
-              v4 != nullptr ? v4 + rec * V4_BYTES : nullptr, vn, v8s != nullptr ? v8s + rec * D : nullptr, vsum);
+  static_assert(sizeof(stage) >= 2 * BN * D && sizeof(stage) >= BN * EXACT_VP * 2, "staging");
+  const int tiles = (a.t + BN - 1) / BN;
+  int wg = blockIdx.x;
+  if (wg < a.krec_wgs) {
+    const int hb = wg / a.chunks, j0 = (wg % a.chunks) * a.per, j1 = min(tiles, j0 + a.per);
+    const int hd = hb % a.hk, b = hb / a.hk;
+    const uint16_t* src = a.k + b * a.ksb + hd * a.ksh;
+    KRaw cur, nxt;
+    load_k_tile(cur, src + (int64_t)j0 * BN * a.kst, a.kst, a.t - j0 * BN);
+    head_stats(a.kpart + (int64_t)hb * STAT_BLOCKS * 3 * D, a.t, j0 == 0, mean, inv, hi, lo,
+               j0 == 0 ? a.kstat + (int64_t)hb * 3 * D : nullptr);
+    auto* c8 = reinterpret_cast<uint8_t (*)[D]>(&stage[0][0]);
+    for (int j = j0; j < j1; ++j) {
+      const int64_t rec = (int64_t)hb * tiles + j;
+      if (j + 1 < j1) load_k_tile(nxt, src + (int64_t)(j + 1) * BN * a.kst, a.kst, a.t - (j + 1) * BN);
+      if (j > j0) __syncthreads();  // (the previous tile's codes are read)
+      quantize_k_tile(cur, a.t - j * BN, mean, a.k8 + rec * K8_BYTES, a.ka + rec * 4,
+                      a.k4 != nullptr ? a.k4 + rec * K4_BYTES : nullptr, a.k4 != nullptr ? a.ka4 + rec * 4 : nullptr, c8,
+                      c8 + BN, a.k4x != nullptr ? a.k4x + rec * K8_BYTES : nullptr);
+      cur = nxt;
+    }
+    return;
+  }
+  wg -= a.krec_wgs;
+  if (wg < a.vrec_wgs) {
+    const int hb = wg / a.chunks, j0 = (wg % a.chunks) * a.per, j1 = min(tiles, j0 + a.per);
+    const int hd = hb % a.hk, b = hb / a.hk;
+    const uint16_t* src = a.v + b * a.vsb + hd * a.vsh;
+    VRaw cur, nxt;
+    load_v_tile(cur, src + (int64_t)j0 * BN * a.vst, a.vst, a.t - j0 * BN);
+    float* stat = j0 == 0 ? a.vstat + (int64_t)hb * 3 * D : nullptr;
+    if (!a.v_identity) {
+      head_stats(a.vpart + (int64_t)hb * STAT_BLOCKS * 3 * D, a.t, true, mean, inv, hi, lo, stat);
+    } else {
+      if (threadIdx.x < D) {
+        mean[threadIdx.x] = 0.f;
+        inv[threadIdx.x] = 1.f;
+        if (stat != nullptr) {
+          stat[threadIdx.x] = 0.f;
+          stat[D + threadIdx.x] = 1.f;
+          stat[2 * D + threadIdx.x] = 1.f;
+        }
+      }
+      __syncthreads();
+    }
+    for (int j = j0; j < j1; ++j) {
+      const int64_t rec = (int64_t)hb * tiles + j;
+      if (j + 1 < j1) load_v_tile(nxt, src + (int64_t)(j + 1) * BN * a.vst, a.vst, a.t - (j + 1) * BN);
+      if (j > j0) __syncthreads();  // (the previous tile's values and sums are read)
+      pack_v_tile(cur, a.t - j * BN, mean, inv, a.v16 != nullptr ? a.v16 + rec * V16_BYTES : nullptr,
+                  a.v8 != nullptr ? a.v8 + rec * V8_BYTES : nullptr, a.v4 != nullptr ? a.v4 + rec * V4_BYTES : nullptr,
+                  stage, a.v8s != nullptr ? a.v8s + rec * D : nullptr, vsum);
+      cur = nxt;
+    }
+    return;
+  }
+  wg -= a.vrec_wgs;
+  // exact heads: workgroup (KV head, tile) of sequence b; other heads leave
+  const int tile = wg % tiles, kh = (wg / tiles) % a.hk, b = wg / (tiles * a.hk);
+  const int slot = a.exact[kh * (a.hq / a.hk)] - 1;
+  if (slot < 0 || slot >= a.nx) return;
+  const int64_t rec = ((int64_t)b * a.nx + slot) * tiles + tile;
+  pack_exact_tile(a.k + b * a.ksb + kh * a.ksh + (int64_t)tile * BN * a.kst, a.kst,
+                  a.v + b * a.vsb + kh * a.vsh + (int64_t)tile * BN * a.vst, a.vst, a.t - tile * BN,
+                  a.kx + rec * KX_BYTES, a.vx + rec * KX_BYTES, reinterpret_cast<uint16_t*>(&stage[0][0]));
 }
 
 }  // namespace tri

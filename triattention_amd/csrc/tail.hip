@@ -119,10 +119,14 @@ __global__ __launch_bounds__(SPILL_THREADS) void tail_spill_kernel(SpillArgs a) 
       const int64_t ks = (int64_t)gr.y + k, vs = (int64_t)gr.z + k;
       if (ks < (is4 ? a.n_k4 : a.n_k8) && vs < a.n_v8 && (!is4 || (a.k4c != nullptr && a.ka4 != nullptr))) {
         float* kap = (is4 ? a.ka4 : a.ka) + (hb * a.tiles_max + j) * 4;
-        quantize_k_tile(kt, a.tst, BN, a.kstat + hb * 3 * D, is4 ? nullptr : a.k8c + ks * K8_BYTES, kap,
+        KRaw kraw;
+        VRaw vraw;
+        load_k_tile(kraw, kt, a.tst, BN);
+        load_v_tile(vraw, vt, a.tst, BN);
+        quantize_k_tile(kraw, BN, a.kstat + hb * 3 * D, is4 ? nullptr : a.k8c + ks * K8_BYTES, kap,
                         is4 ? a.k4c + ks * K4_BYTES : nullptr, kap, sm.q.c8, sm.q.c4);
         const float* vm = a.vstat + hb * 3 * D;
-        pack_v_tile(vt, a.tst, BN, vm, vm + 2 * D, nullptr, a.v8c + vs * V8_BYTES, nullptr, sm.q.vn);
+        pack_v_tile(vraw, BN, vm, vm + 2 * D, nullptr, a.v8c + vs * V8_BYTES, nullptr, sm.q.vn);
         __syncthreads();  // the four group scales are written (lane 0 of each wave)
         if (tid == 0) {
           const int info = (gr.x & 0x1ff) | (int)((uint32_t)ks << 9);

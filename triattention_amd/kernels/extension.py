@@ -36,7 +36,7 @@ D = 128
 STAT_BLOCKS = 64
 K8_WORDS, K4_WORDS, V16_WORDS, V8_WORDS, V4_WORDS = 2048, 1024, 4096, 2048, 1024
 
-EXPORTS = ("tri_last_error", "tri_prepare_qk", "tri_pack_v", "tri_attention", "tri_pack_exact", "tri_decode",
+EXPORTS = ("tri_last_error", "tri_prepare_qk", "tri_pack_v", "tri_prepare", "tri_attention", "tri_pack_exact", "tri_decode",
            "tri_decode_partials", "tri_decode_merge", "tri_decode_short_tail", "tri_decode_merge_short_tail",
            "tri_decode_partials_timed", "tri_decode_noalloc",
            "tri_decode_tasks", "tri_cache_store", "tri_tail_spill", "tri_decode_occupancy", "tri_device_cus",
@@ -62,6 +62,7 @@ def load_library() -> ctypes.CDLL:
     lib.tri_prepare_qk.argtypes = [P, I64, I64, I64, P, I64, I64, I64, I, I, I, I,
                                    P, P, P, P, P, P, P, P, P, P, P, P]
     lib.tri_pack_v.argtypes = [P, I64, I64, I64, I, I, I, P, P, P, P, P, P, P]
+    lib.tri_prepare.argtypes = ([P, I64, I64, I64] * 3 + [I, I, I, I] + [P] * 11 + [P] * 6 + [P, I, P, P, P])
     lib.tri_attention.argtypes = [P, I, P, I, I, I, I, P, P, P, P, P, P, P, P, P, P, P, P, I, I64, I64, I64, D_,
                                   P, P, I64, I64, I64, P, P, I, P, P, P]
     lib.tri_pack_exact.argtypes = [P, I64, I64, I64, P, I64, I64, I64, I, I, I, I, P, I, P, P, P]
@@ -106,7 +107,7 @@ def _check(cond: bool, message: str) -> None:
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 class Module:
@@ -123,15 +124,12 @@ class Module:
             raise RuntimeError(self.lib.tri_last_error().decode())
 
     @staticmethod
-    def _stream(device) -> ctypes.c_void_p:
-        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    def _stream(device) -> int:
+        return torch.cuda.current_stream(device).cuda_stream
 
     # -------------------------------------------------------------- prepare_qk
-    def prepare_qk(self, q, k, q8, qa, kp, ka, partial, kstat, q4=None, qa4=None, k4p=None, ka4=None, k4x=None):
-        """Per-token INT8 (and INT4) Q and centred per-block INT8 (and INT4) K operands.
-
-        Extension: ``k4x`` (uint32, as many words as ``kp``, with the INT4 buffers) receives the K4 records
-        expanded to 16 * code bytes in the K8 layout, which ``attention(..., k4x=...)`` reads."""
+    @staticmethod
+    def _check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x):
         _check(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 4 and q.size(3) == D and q.stride(3) == 1 and
                k.dtype == torch.bfloat16 and k.dim() == 4 and k.size(0) == q.size(0) and k.size(2) == q.size(2) and
                k.size(3) == D and k.stride(3) == 1, "BF16 Q/K [B,H,T,128] with contiguous features")
@@ -148,6 +146,40 @@ class Module:
                "INT4 Q/K buffers (all or none)")
         _check(k4x is None or (int4 and k4x.dtype == torch.uint32 and k4x.is_contiguous() and
                                k4x.numel() == b * hk * tiles * K8_WORDS), "expanded K4 records (with the INT4 buffers)")
+        return b, hq, hk, t
+
+    @staticmethod
+    def _check_v(v, partial, vstat, v16p, v8p, v4p, v8sum):
+        _check(v.is_cuda and v.dtype == torch.bfloat16 and v.dim() == 4 and v.size(3) == D and v.stride(3) == 1,
+               "BF16 V [B,Hkv,T,128]")
+        b, hk, t, _ = v.shape
+        tiles = (t + 63) // 64
+        _check(partial.numel() >= b * hk * STAT_BLOCKS * 3 * D and vstat.numel() == b * hk * 3 * D,
+               "V statistics buffers")
+        for x, words in ((v16p, V16_WORDS), (v8p, V8_WORDS), (v4p, V4_WORDS)):
+            _check(x is None or (x.dtype == torch.uint32 and x.is_contiguous() and x.numel() == b * hk * tiles * words),
+                   "packed V size")
+        _check(v8sum is None or (v8p is not None and _v8sum_ok(v8sum, b * hk * tiles)), "V8 sums")
+        return b, hk, t
+
+    @staticmethod
+    def _check_exact(k, v, exact, nx, kx, vx):
+        _check(k.dtype == v.dtype == torch.bfloat16 and k.dim() == 4 and k.shape == v.shape and k.size(3) == D and
+               k.stride(3) == 1 and v.stride(3) == 1, "K/V bf16 [B,Hk,T,128]")
+        b, hk, t, _ = k.shape
+        h = exact.numel()
+        tiles = (t + 63) // 64
+        _check(exact.dtype == torch.int32 and exact.is_cuda and h % hk == 0, "exact flags [Hq]")
+        _check(1 <= nx <= hk and kx.numel() * kx.element_size() >= b * nx * tiles * KX_BYTES and
+               vx.numel() * vx.element_size() >= b * nx * tiles * KX_BYTES, "KX/VX records [B][nx][tiles]")
+        return b, h, hk, t
+
+    def prepare_qk(self, q, k, q8, qa, kp, ka, partial, kstat, q4=None, qa4=None, k4p=None, ka4=None, k4x=None):
+        """Per-token INT8 (and INT4) Q and centred per-block INT8 (and INT4) K operands.
+
+        Extension: ``k4x`` (uint32, as many words as ``kp``, with the INT4 buffers) receives the K4 records
+        expanded to 16 * code bytes in the K8 layout, which ``attention(..., k4x=...)`` reads."""
+        b, hq, hk, t = self._check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x)
         with torch.cuda.device(q.device):
             self._call(self.lib.tri_prepare_qk, _ptr(q), q.stride(0), q.stride(1), q.stride(2), _ptr(k), k.stride(0),
                        k.stride(1), k.stride(2), b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka), _ptr(partial),
@@ -159,19 +191,27 @@ class Module:
 
         Extension: ``v8sum`` (int32 [B*Hkv*tiles*128], with ``v8p``) receives -127 times each channel's
         sum of each tile's V8 codes, which ``attention(..., v8sum=...)`` starts its P V products from."""
-        _check(v.is_cuda and v.dtype == torch.bfloat16 and v.dim() == 4 and v.size(3) == D and v.stride(3) == 1,
-               "BF16 V [B,Hkv,T,128]")
-        b, hk, t, _ = v.shape
-        tiles = (t + 63) // 64
-        _check(partial.numel() >= b * hk * STAT_BLOCKS * 3 * D and vstat.numel() == b * hk * 3 * D,
-               "V statistics buffers")
-        for x, words in ((v16p, V16_WORDS), (v8p, V8_WORDS), (v4p, V4_WORDS)):
-            _check(x is None or (x.dtype == torch.uint32 and x.is_contiguous() and x.numel() == b * hk * tiles * words),
-                   "packed V size")
-        _check(v8sum is None or (v8p is not None and _v8sum_ok(v8sum, b * hk * tiles)), "V8 sums")
+        b, hk, t = self._check_v(v, partial, vstat, v16p, v8p, v4p, v8sum)
         with torch.cuda.device(v.device):
             self._call(self.lib.tri_pack_v, _ptr(v), v.stride(0), v.stride(1), v.stride(2), b, hk, t, _ptr(partial),
                        _ptr(vstat), _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum), self._stream(v.device))
+
+    # ----------------------------------------------------------------- prepare
+    def prepare(self, q, k, v, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x, vpartial, vstat, v16p, v8p,
+                v4p, v8sum, exact=None, nx=0, kx=None, vx=None):
+        """``prepare_qk``, ``pack_v`` and (with ``exact``) ``pack_exact`` of one prompt in two launches
+        (extension): the same buffers with the same contents, K's and V's statistics partials in
+        scratch buffers of their own."""
+        b, hq, hk, t = self._check_qk(q, k, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x)
+        _check(self._check_v(v, vpartial, vstat, v16p, v8p, v4p, v8sum) == (b, hk, t), "V [B,Hkv,T,128] like K")
+        if exact is not None:
+            _check(self._check_exact(k, v, exact, nx, kx, vx)[1] == hq, "exact flags [Hq]")
+        with torch.cuda.device(q.device):
+            self._call(self.lib.tri_prepare, _ptr(q), *q.stride()[:3], _ptr(k), *k.stride()[:3], _ptr(v),
+                       *v.stride()[:3], b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka), _ptr(kpartial),
+                       _ptr(kstat), _ptr(q4), _ptr(qa4), _ptr(k4p), _ptr(ka4), _ptr(k4x), _ptr(vpartial), _ptr(vstat),
+                       _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum), _ptr(exact), int(nx), _ptr(kx), _ptr(vx),
+                       self._stream(q.device))
 
     # --------------------------------------------------------------- attention
     def attention(self, order, bands, groups, entries, v16p, v8p, v4p, vstat, q8, k8p, qa8, ka8, q4, k4p, qa4, ka4,
@@ -222,14 +262,7 @@ class Module:
 
     def pack_exact(self, k, v, exact, nx, kx, vx):
         """bf16 K/V of the exact KV heads -> KX/VX records [B][nx][tiles] (16 KiB each; extension)."""
-        _check(k.dtype == v.dtype == torch.bfloat16 and k.dim() == 4 and k.shape == v.shape and k.size(3) == D and
-               k.stride(3) == 1 and v.stride(3) == 1, "K/V bf16 [B,Hk,T,128]")
-        b, hk, t, _ = k.shape
-        h = exact.numel()
-        tiles = (t + 63) // 64
-        _check(exact.dtype == torch.int32 and exact.is_cuda and h % hk == 0, "exact flags [Hq]")
-        _check(1 <= nx <= hk and kx.numel() * kx.element_size() >= b * nx * tiles * KX_BYTES and
-               vx.numel() * vx.element_size() >= b * nx * tiles * KX_BYTES, "KX/VX records [B][nx][tiles]")
+        b, h, hk, t = self._check_exact(k, v, exact, nx, kx, vx)
         with torch.cuda.device(k.device):
             self._call(self.lib.tri_pack_exact, _ptr(k), *k.stride()[:3], _ptr(v), *v.stride()[:3], b, h, hk, t,
                        _ptr(exact), int(nx), _ptr(kx), _ptr(vx), self._stream(k.device))

@@ -1,5 +1,5 @@
 """Prefill host operator: band table, scratch pool and the op sequence
-``prepare_qk -> pack_v -> attention -> store``.
+``prepare_qk -> pack_v -> attention -> store`` (the first two, and ``pack_exact``, as one ``prepare`` call).
 
 Mirrors triattention/kernels/prefill.py (BandTable :10-28, Prefill :31-108)
 with the same names, call signature and buffer-sharing contract, extended to a
@@ -82,6 +82,7 @@ SCRATCH = (
     ("k", lambda L: L.batch * L.hk * L.tiles * 2048, torch.uint32, lambda L: True),
     ("ka", lambda L: L.batch * L.hk * L.tiles * 4, torch.float32, lambda L: True),
     ("partial", lambda L: L.batch * L.hk * 64 * 3 * 128, torch.float32, lambda L: True),
+    ("vpartial", lambda L: L.batch * L.hk * 64 * 3 * 128, torch.float32, lambda L: True),
     ("kstat", lambda L: L.batch * L.hk * 3 * 128, torch.float32, lambda L: True),
     ("vstat", lambda L: L.batch * L.hk * 3 * 128, torch.float32, lambda L: True),
     ("q4", lambda L: L.batch * L.hq * L.t * 64, torch.uint8, lambda L: L.int4),
@@ -198,7 +199,7 @@ class Prefill:
         self._run(layer, q, k, v, None, attend=False)
 
     def _run(self, layer, q, k, v, scale, attend):
-        """The reference's op sequence (kernels/prefill.py:87-108): quantize Q/K, pack V, attend,
+        """The reference's op sequence (kernels/prefill.py:87-108): quantize Q/K and pack V (``prepare``), attend,
         then hand the records to the decode cache."""
         batch, hq, t, _ = q.shape
         hk, rows, device = k.shape[1], (t + 63) // 64, q.device
@@ -209,15 +210,14 @@ class Prefill:
         ops = self.operands(layout, device)
         packed = ops["packed"]
         k4x = ops["k4x"] if attend else None  # (only the prompt's attention reads the expanded records)
-        self.module.prepare_qk(q, k, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"],
-                               ops["q4"], ops["qa4"], ops["k4"], ops["ka4"], k4x=k4x)
         v8sum = ops["v8sum"] if attend else None  # (only the prompt's attention reads the sums)
-        self.module.pack_v(v, ops["partial"], ops["vstat"], packed[F16], packed[I8], packed[I4], v8sum=v8sum)
         exact, nx = self.exact(layer, hq, hk, device)
         kx = vx = None
         if exact is not None:
             kx, vx = self.exact_records(batch * nx * rows * KX_BYTES, device)
-            self.module.pack_exact(k, v, exact, nx, kx, vx)
+        self.module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"],
+                            ops["q4"], ops["qa4"], ops["k4"], ops["ka4"], k4x, ops["vpartial"], ops["vstat"],
+                            packed[F16], packed[I8], packed[I4], v8sum, exact, nx, kx, vx)
         out = None
         if attend:
             dtype = self.out_dtype or q.dtype
