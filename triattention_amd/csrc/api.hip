@@ -67,6 +67,18 @@ static void launch_decode(int g, dim3 grid, const tri::DecodeArgs& d, hipStream_
   }
 }
 
+// The same for caches that hold exact (bf16) heads: one wave per workgroup.
+template <bool T>
+static void launch_decode_exact(int g, dim3 grid, const tri::DecodeArgs& d, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+  switch (g) {
+    case 1: launch_one<1>(tri::decode_kernel<1, true, true, 1, 2, T>, grid, d, s, e0, e1); break;
+    case 2: launch_one<1>(tri::decode_kernel<2, true, true, 1, 2, T>, grid, d, s, e0, e1); break;
+    case 3: launch_one<1>(tri::decode_kernel<3, true, true, 1, 2, T>, grid, d, s, e0, e1); break;
+    case 4: launch_one<1>(tri::decode_kernel<4, true, true, 1, 2, T>, grid, d, s, e0, e1); break;
+    default: launch_one<1>(tri::decode_kernel<4, true, false, 1, 2, T>, grid, d, s, e0, e1); break;
+  }
+}
+
 // CU count of the current device, cached per device (devices 0..63)
 static int device_cus(int* cus) {
   static std::atomic<int> cached[64];
@@ -409,8 +421,7 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
   d.maxn = maxn;
   d.per = per;
   d.bounds = bounds;
-  // a task table lists the splits to run (exact heads gather their splits themselves)
-  d.tasks = xslot == nullptr ? static_cast<const int32_t*>(tasks) : nullptr;
+  d.tasks = static_cast<const int32_t*>(tasks);  // (lists the splits to run)
   if (d.tasks && (n_tasks < 1 || !aligned(tasks, 16))) return fail("decode: a task table needs n_tasks >= 1, 16-byte aligned");
   d.tiles_max = tiles_max;
   d.splits = splits;
@@ -517,20 +528,16 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
         else launch_decode<1, false>(g, grid, d, s, ev_start, ev_stop);
       }
     } else {
-      // groups of up to 4 q-heads use the DUP lane layout (both wave halves on rows 0..3)
-      switch (g) {
-        case 1: launch_one<1>(tri::decode_kernel<1, true, true>, grid, d, s, ev_start, ev_stop); break;
-        case 2: launch_one<1>(tri::decode_kernel<2, true, true>, grid, d, s, ev_start, ev_stop); break;
-        case 3: launch_one<1>(tri::decode_kernel<3, true, true>, grid, d, s, ev_start, ev_stop); break;
-        case 4: launch_one<1>(tri::decode_kernel<4, true, true>, grid, d, s, ev_start, ev_stop); break;
-        default: launch_one<1>(tri::decode_kernel<4, true, false>, grid, d, s, ev_start, ev_stop); break;
-      }
+      if (d.tasks) launch_decode_exact<true>(g, grid, d, s, ev_start, ev_stop);
+      else launch_decode_exact<false>(g, grid, d, s, ev_start, ev_stop);
     }
   }
   if (phase & 2) {
     // phase bit 4: the merge as one wave per (sequence, q-head), for short tails
     if (phase & 4) tri::decode_merge1_kernel<<<dim3(hq, batch), 64, 0, s>>>(mg);
-    else tri::decode_merge_kernel<<<dim3(hq, batch), 256, 0, s>>>(mg);
+    // (a narrow grid's form does not depend on the tail: no choice on the device)
+    else if (mg.wide) tri::decode_merge_kernel<<<dim3(hq, batch), 256, 0, s>>>(mg);
+    else tri::decode_merge_narrow_kernel<tri::MERGE_NARROW><<<dim3(hq, batch), 64 * tri::MERGE_NARROW, 0, s>>>(mg);
   }
   return check_launch("decode");
 }
@@ -646,7 +653,7 @@ int tri_decode_noalloc(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
   float* pm = s;
   float* pl = s + pad;
   float* po = s + 2 * pad;
-  if (tasks && xslot == nullptr) {
+  if (tasks) {
     // splits a task table leaves out are never written: the scratch (which holds whatever the last
     // call left) gets the empty partial in every slot first
     tri::fill_empty_partials_kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, hs>>>(pm, pl, po, n);

@@ -161,14 +161,14 @@ __device__ __forceinline__ v4i unpack16(v4i w) {
 // softmax, P split into bf16 high and low parts, O^T = V^T P^T.  The partials
 // use the quantized heads' convention: m in log2 units, l = sum p, o = sum p v'
 // with v' = (v - mean) / scale, so the merge treats every head alike.
-__device__ __forceinline__ void decode_exact(const DecodeArgs& a, int b, int kh, int split) {
+// (The first records load after Q is read: issued before it, the split kernel measured 5-10% slower, 15.1 against
+// 16.9 us on 8 sequences of 4,096 tokens, 4 exact KV heads.)
+__device__ __forceinline__ void decode_exact(const DecodeArgs& a, int b, int kh, int split, int first, int last) {
   // Q as the B operand, kept in LDS: column lq = q-head kh*g + lq, features ks*16 + 8*half + e
   __shared__ __align__(16) uint16_t qx[32][D];
   const int L = threadIdx.x, lq = L & 31, half = L >> 5;
   const int g = a.hq / a.hk, prompt = a.prompt[b], ptiles = (prompt + BN - 1) / BN;
   const int64_t hb = (int64_t)b * a.hk + kh;
-  int first, last;
-  split_range(a, hb, split, first, last);
   const int x0 = a.xslot[hb];
   float cq = 0.f;
   const float* kmean = a.kstat + hb * 3 * D;
@@ -285,14 +285,12 @@ __device__ __forceinline__ void decode_exact(const DecodeArgs& a, int b, int kh,
 // quantization and metadata, take its tiles alternately (wave w: entries first
 // + w, first + w + 2, ...), and combine their running (m, l, o) in LDS at the
 // end, so that each SIMD holds two waves whose dependency chains interleave.
-// TASKS: the launch has a task table (a.tasks, quantized heads only), whose rows give each split's
-// entries; a separate instantiation, so that the common path has no branch between the first
+// TASKS: the launch has a task table (a.tasks), whose rows give each split's entries; a separate instantiation, so that the common path has no branch between the first
 // tile's record loads and the use of Q (at a join of two paths the compiler waits for every
 // outstanding load, which would hold the Q quantization until the records arrive).
 template <int R, bool EXACT = false, bool DUP = false, int NW = 1, int W = 2, bool TASKS = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(W))) void decode_kernel(DecodeArgs a) {
   static_assert(NW == 1 || (NW == 2 && !EXACT), "two waves per workgroup only for quantized heads");
-  static_assert(!(TASKS && EXACT), "task tables list quantized heads only");
   __shared__ __align__(16) int8_t q8s[MAX_GROUP][D];
   __shared__ __align__(16) int8_t q4s[MAX_GROUP][D];
   __shared__ float qsc[MAX_GROUP], qsc4[MAX_GROUP];
@@ -349,7 +347,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(W))) vo
   }
   if constexpr (EXACT) {
     if (a.xslot[(int64_t)b * a.hk + kh] >= 0) {
-      decode_exact(a, b, kh, split);
+      // (a task row's entries are tiles: an exact head keeps every one, so entry 0's tile is the first)
+      if constexpr (TASKS) {
+        first = (int)((unsigned)__builtin_amdgcn_readlane(task_w.z, 0) >> 10);
+        last += first;
+      }
+      decode_exact(a, b, kh, split, first, last);
       return;
     }
   }
@@ -861,19 +864,28 @@ struct MergeArgs {
 };
 
 // LSE merge of the split partials with the exact bf16 tail
-// (common_device.cuh:373-469).  One 256-thread workgroup per (sequence, q-head),
+// (common_device.cuh:373-469).  One workgroup of NW waves per (sequence, q-head),
 // XCD-aware so the q-heads of one KV head share an L2 for their tail reads.
 // Every global load that does not depend on another is issued first (the split
-// partials of up to 16 splits, the first 32 tail tokens' K rows and first 64
+// partials of up to 64 splits, the first 32 tail tokens' K rows and first 64
 // tail tokens' V rows), so a short tail costs one memory round trip; longer
-// tails and more splits continue in loops.  Tail scores: 8 lanes per token (16
+// tails and more splits continue in loops that keep MERGE_K rounds of 32 K rows and
+// MERGE_V rounds of 16 V rows in flight.  Tail scores: 8 lanes per token (16
 // channels each); tail values: 16 lanes per token (8 channels each).
-__device__ __forceinline__ void merge_four(const MergeArgs& a) {
+constexpr int MERGE_K = 2, MERGE_V = 4;
+// Waves per (sequence, q-head) on grids of fewer than SHORT_WIDE workgroups per CU, which leave SIMDs idle:
+// a long tail is bound by each wave's own scores and weights.  Kernel times at 4 / 8 / 16 waves: 256
+// workgroups, 700-token tails 16.9 / 11.7 / 12.0 us (19.9 with one round of K rows in flight and the splits past 16
+// one after another); 28 workgroups, 64 splits, 37-token tails 5.3 / 4.6 / 6.1 us (8.0).
+constexpr int MERGE_NARROW = 8;
+template <int NW>
+__device__ __forceinline__ void merge_waves(const MergeArgs& a) {
+  constexpr int SG = 8 * NW, VG = 4 * NW;  // token groups of the score and value layouts
   __shared__ float ts[MAX_TAIL];  // tail scores
-  __shared__ float vo[16][D];     // tail value sums of the 16 token groups
-  __shared__ float wo[4][D];      // split sums of the four waves
-  __shared__ float wred[4][2];    // per wave: max, split weight sum
-  __shared__ float ltg[16];       // tail weight sums of the 16 token groups
+  __shared__ float vo[VG][D];     // tail value sums of the token groups
+  __shared__ float wo[NW][D];     // split sums of the waves
+  __shared__ float wred[NW][2];   // per wave: max, split weight sum
+  __shared__ float ltg[VG];       // tail weight sums of the token groups
   int hq, b;
   {
     const int total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
@@ -904,27 +916,40 @@ __device__ __forceinline__ void merge_four(const MergeArgs& a) {
     qv[i] = bf16f(a.q[b * a.qsb + hq * a.qsh + sc0 + i]);
     mu[i] = a.kstat[hb * 3 * D + sc0 + i];
   }
+  // tail rows through the current token's (clamped to the last one: lanes past the tail load it again)
+  auto krow = [&](int t, uint4 (&raw)[2]) {
+    const int tt = min(t, tail - 1);
+    const uint16_t* row = (tt < prior ? kt + (int64_t)tt * a.tst : kc) + sc0;
+    raw[0] = *reinterpret_cast<const uint4*>(row);
+    raw[1] = *reinterpret_cast<const uint4*>(row + 8);
+  };
+  auto vrow = [&](int t) {
+    const int tt = min(t, tail - 1);
+    return *reinterpret_cast<const uint4*>((tt < prior ? vt + (int64_t)tt * a.tst : vc) + vc0);
+  };
   uint4 kraw[2];
-  {
-    const int t = min(sgrp, tail - 1);
-    const uint16_t* row = (t < prior ? kt + (int64_t)t * a.tst : kc) + sc0;
-    kraw[0] = *reinterpret_cast<const uint4*>(row);
-    kraw[1] = *reinterpret_cast<const uint4*>(row + 8);
-  }
+  krow(sgrp, kraw);
   uint4 vraw[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int t = min(vgrp + u * 16, tail - 1);
-    vraw[u] = *reinterpret_cast<const uint4*>((t < prior ? vt + (int64_t)t * a.tst : vc) + vc0);
-  }
-  float pmv[4], plv[4];
-  float2 pov[4];
+  for (int u = 0; u < 4; ++u) vraw[u] = vrow(vgrp + u * VG);
+  // split partials: lane s of every wave holds (m, l) of split s, wave w the values of splits w, w + NW, ...
+  // below 64 (the rows a caller has no splits for are not read)
+  const int splits = a.splits;
+  const float pms = lane < splits ? a.pm[pbase + lane] : -3.402823466e38f;
+  const float pls = lane < splits ? a.pl[pbase + lane] : 0.f;
+  const int swave = __builtin_amdgcn_readfirstlane(wave);
+  auto split_o = [&](int s) { return *reinterpret_cast<const float2*>(a.po + (pbase + s) * D + lane * 2); };
+  constexpr int SU = 64 / NW;  // rounds of the first 64 splits
+  float2 pov[SU];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int s = min(wave + 4 * u, a.splits - 1);
-    pmv[u] = a.pm[pbase + s];
-    plv[u] = a.pl[pbase + s];
-    pov[u] = *reinterpret_cast<const float2*>(a.po + (pbase + s) * D + lane * 2);
+  for (int u = 0; u < SU / 4; ++u) pov[u] = split_o(min(swave + NW * u, splits - 1));
+  if (splits > 16) {
+#pragma unroll
+    for (int u = SU / 4; u < SU / 2; ++u) pov[u] = split_o(min(swave + NW * u, splits - 1));
+  }
+  if (splits > 32) {
+#pragma unroll
+    for (int u = SU / 2; u < SU; ++u) pov[u] = split_o(min(swave + NW * u, splits - 1));
   }
   const float vmv = tid < D ? vmean[tid] : 0.f, vsv = tid < D ? vscale[tid] : 0.f;
   if (hq % g == 0 && tid < D) {
@@ -946,39 +971,42 @@ __device__ __forceinline__ void merge_four(const MergeArgs& a) {
     if ((tid & 7) == 0 && t < tail) ts[t] = part * a.sm_log2;
   };
   score(kraw, sgrp);
-  for (int t0 = sgrp + 32; t0 < tail; t0 += 32) {
-    const int t = min(t0, tail - 1);
-    const uint16_t* row = (t < prior ? kt + (int64_t)t * a.tst : kc) + sc0;
-    uint4 raw[2] = {*reinterpret_cast<const uint4*>(row), *reinterpret_cast<const uint4*>(row + 8)};
-    score(raw, t0);
-  }
-  float pm_own = -3.402823466e38f;
+  // MERGE_K rounds of SG tokens in flight
+  for (int t0 = SG; t0 < tail; t0 += SG * MERGE_K) {
+    uint4 raw[MERGE_K][2];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (wave + 4 * u < a.splits) pm_own = fmaxf(pm_own, pmv[u]);
-  for (int s = wave + 16; s < a.splits; s += 4) pm_own = fmaxf(pm_own, a.pm[pbase + s]);
+    for (int u = 0; u < MERGE_K; ++u)
+      krow(t0 + SG * u + sgrp, raw[u]);
+#pragma unroll
+    for (int u = 0; u < MERGE_K; ++u)
+      score(raw[u], t0 + SG * u + sgrp);
+  }
+  float pm_own = pms;
+  for (int s = 64 + lane; s < splits; s += 64) pm_own = fmaxf(pm_own, a.pm[pbase + s]);
   __syncthreads();
   float m = pm_own;
-  for (int t = tid; t < tail; t += 256) m = fmaxf(m, ts[t]);
+  for (int t = tid; t < tail; t += 64 * NW) m = fmaxf(m, ts[t]);
   m = wave_max(m);
   if (lane == 0) wred[wave][0] = m;
   __syncthreads();
-  m = fmaxf(fmaxf(wred[0][0], wred[1][0]), fmaxf(wred[2][0], wred[3][0]));
-  // split sums: wave w takes splits w, w + 4, ... in order
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m = fmaxf(m, wred[w][0]);
+  // split sums: wave w takes splits w, w + NW, ... in order
   float l = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (wave + 4 * u < a.splits) {
-      const float w = texp2(pmv[u] - m);
-      l = __builtin_fmaf(plv[u], w, l);
+  for (int u = 0; u < SU; ++u) {
+    const int sp = swave + NW * u;
+    if (sp < splits) {
+      const float w = texp2(readlane_f(pms, sp) - m);
+      l = __builtin_fmaf(readlane_f(pls, sp), w, l);
       o0 = __builtin_fmaf(pov[u].x, w, o0);
       o1 = __builtin_fmaf(pov[u].y, w, o1);
     }
   }
-  for (int s = wave + 16; s < a.splits; s += 4) {
+  for (int s = swave + 64; s < splits; s += NW) {
     const float w = texp2(a.pm[pbase + s] - m);
     l = __builtin_fmaf(a.pl[pbase + s], w, l);
-    const float2 p = *reinterpret_cast<const float2*>(a.po + (pbase + s) * D + lane * 2);
+    const float2 p = split_o(s);
     o0 = __builtin_fmaf(p.x, w, o0);
     o1 = __builtin_fmaf(p.y, w, o1);
   }
@@ -998,16 +1026,16 @@ __device__ __forceinline__ void merge_four(const MergeArgs& a) {
       for (int i = 0; i < 8; ++i) av[i] = __builtin_fmaf(e, bf16f((uint16_t)(w[i >> 1] >> (16 * (i & 1)))), av[i]);
     };
 #pragma unroll
-    for (int u = 0; u < 4; ++u) accum(vraw[u], vgrp + u * 16);
-    for (int t0 = vgrp + 64; t0 < tail; t0 += 4 * 16) {
-      uint4 raw[4];
+    for (int u = 0; u < 4; ++u) accum(vraw[u], vgrp + u * VG);
+    // MERGE_V rounds of VG tokens in flight
+    for (int t0 = 4 * VG; t0 < tail; t0 += VG * MERGE_V) {
+      uint4 raw[MERGE_V];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = min(t0 + u * 16, tail - 1);
-        raw[u] = *reinterpret_cast<const uint4*>((t < prior ? vt + (int64_t)t * a.tst : vc) + vc0);
-      }
+      for (int u = 0; u < MERGE_V; ++u)
+        raw[u] = vrow(t0 + VG * u + vgrp);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) accum(raw[u], t0 + u * 16);
+      for (int u = 0; u < MERGE_V; ++u)
+        accum(raw[u], t0 + VG * u + vgrp);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) vo[vgrp][vc0 + i] = av[i];
@@ -1017,12 +1045,12 @@ __device__ __forceinline__ void merge_four(const MergeArgs& a) {
   if (tid >= D) return;
   float lsum = 0.f, osum = 0.f, tsum = 0.f, vsum = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < NW; ++w) {
     lsum += wred[w][1];
     osum += wo[w][tid];
   }
 #pragma unroll
-  for (int grp = 0; grp < 16; ++grp) {
+  for (int grp = 0; grp < VG; ++grp) {
     vsum += vo[grp][tid];
     tsum += ltg[grp];
   }
@@ -1229,7 +1257,7 @@ __device__ __forceinline__ int merge_tail(const MergeArgs& a) {
 
 // The merge with the form chosen on the device: one wave (merge_one, the reference's order) while
 // the tail holds at most SHORT_TAIL tokens on a grid of at least SHORT_WIDE workgroups per CU (a.wide),
-// four waves (merge_four) otherwise.  Measured (kernel durations, Hq 28): on 896 workgroups the one-wave
+// four waves (merge_waves<4>) otherwise.  Measured (kernel durations, Hq 28): on 896 workgroups the one-wave
 // form takes 5.5 / 6.1 / 7.6 / 10.7 us at tails of 4 / 16 / 32 / 64 tokens against 6.8 / 6.8 / 6.8 / 7.6
 // for four waves; on 448 or fewer four waves are as fast or faster at every tail (4.3-5.5 us).  A
 // captured graph replays one launch at steps whose tails grow, so the choice cannot be the host's:
@@ -1242,8 +1270,14 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(MergeArgs a) {
     if (threadIdx.x >= 64) return;
     merge_one(a);
   } else {
-    merge_four(a);
+    merge_waves<4>(a);
   }
+}
+
+// The merge of narrow grids (!a.wide), whose form does not depend on the tail: NW waves per (sequence, q-head).
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void decode_merge_narrow_kernel(MergeArgs a) {
+  merge_waves<NW>(a);
 }
 
 // The one-wave form alone, whatever the tail (tri_decode_short_tail).

@@ -143,22 +143,27 @@ def balanced_partition(metas, batches, slots: int):
     Extension (the reference splits every head into runs of one tile count, decode.py:54-55): the
     split kernel streams each split's records at about the same rate per wave, so its time is set
     by the largest split.  Heads are cut by cost (the measured time of each tile's kind) into
-    n_h = ceil(cost_h / t) runs of near-equal cost, with the smallest target t whose split count
-    fits ``slots`` resident workgroups, at most 64 entries per split."""
+    n_h = min(ceil(cost_h / t), tiles) runs of near-equal cost, with the smallest target t whose split
+    count fits ``slots`` resident workgroups, at most 64 entries per split.  A short cache thus gets one
+    tile per split (4 KV heads of 64 tiles, one exact: 256 one-tile splits)."""
     costs = [entry_costs(m) for m in metas]
     heads = [c.sum(1) for c in costs]
     floors = [np.maximum((m["count"].numpy() + 63) // 64, 1) for m in metas]
     h_all, f_all = np.concatenate(heads), np.concatenate(floors).astype(np.float64)
     w_all = np.concatenate([np.full(len(h), b, np.float64) for h, b in zip(heads, batches)])
-    items = lambda t: float((w_all * np.maximum(np.ceil(h_all / t), f_all)).sum())
-    lo, hi = max(float(c.max()) for c in costs), float(h_all.max()) + 1.0
+    c_all = np.concatenate([m["count"].numpy() for m in metas]).astype(np.float64)
+    items = lambda t: float((w_all * np.maximum(np.minimum(np.ceil(h_all / t), c_all), f_all)).sum())
+    # (no target below the cheapest tile: a head has at most one run per tile)
+    lo, hi = min(float(c[c > 0].min(initial=np.inf)) for c in costs), float(h_all.max()) + 1.0
+    if not np.isfinite(lo):
+        lo = 1.0
     if items(hi) <= slots:
         for _ in range(60):
             mid = (lo + hi) / 2
             lo, hi = (lo, mid) if items(mid) <= slots else (mid, hi)
     out = []
     for m, c, h, f in zip(metas, costs, heads, floors):
-        n = np.maximum(np.ceil(h / hi).astype(np.int64), f)
+        n = np.maximum(np.minimum(np.ceil(h / hi).astype(np.int64), m["count"].numpy()), f)
         valid = m["valid"].numpy()
         while True:
             b = split_bounds(c, valid, n)
