@@ -1,0 +1,60 @@
+"""The decode cache's shared split layouts: by shape and bands, bounded, and equal to a fresh computation."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from cache_host import HostCacheModule
+from triattention_amd.kernels.decode import DecodeCache
+from triattention_amd.kernels.prefill import F16, I4, I8
+from triattention_amd.synthetic import INF
+
+BANDS = torch.tensor([[INF, INF], [1, INF], [2, 4], [1, 1]], dtype=torch.int32)
+
+
+def store(cache, layer, prompt, batch=1, bands=BANDS, value=1.0, hk=2):
+    tiles = (prompt + 63) // 64
+    n = batch * hk * tiles
+    rec = lambda words: torch.full((n * words,), int(value), dtype=torch.int32).view(torch.uint32)
+    scales = torch.full((n * 4,), value)
+    stat = torch.full((batch, hk, 3, 128), value)
+    cache.store(layer, prompt, rec(2048), scales, stat, stat.clone(), {F16: None, I8: rec(2048), I4: rec(1024)},
+                cache.codes(tiles)[0], bands, rec(1024), scales.clone())
+    return cache.layers[layer]
+
+
+def test_prompts_of_one_shape_share_a_layout_and_keep_their_own_data():
+    cache = DecodeCache(HostCacheModule(), max_tail=8)
+    a, b = store(cache, 0, 200, value=1.0), store(cache, 1, 200, value=2.0)
+    assert a["layout"] is b["layout"] and len(cache.layouts) == 1
+    assert a["ka"].data_ptr() != b["ka"].data_ptr()
+    assert bool((a["ka"] == 1).all()) and bool((b["ka"] == 2).all())
+    for e in (a, b):
+        assert not e["tail_k"].any() and not e["tail_v"].any() and e["store"].arrays["tail_base"].tolist() == [0, 0]
+    # the last tile's length, the batch, the bands and a forced split each give a layout of their own
+    assert store(cache, 2, 200, batch=2)["layout"] is not a["layout"]
+    assert store(cache, 3, 264)["layout"] is not a["layout"]
+    assert store(cache, 4, 200, bands=BANDS.flip(0))["layout"] is not a["layout"]
+    cache.per = 1
+    assert store(cache, 5, 200)["layout"]["bounds"] is None
+
+
+@pytest.mark.parametrize("prompt, batch", [(1, 1), (64, 3), (65, 1), (1100, 2), (4000, 1)])
+def test_a_shared_layout_equals_a_fresh_one(prompt, batch):
+    shared = DecodeCache(HostCacheModule(), max_tail=8)
+    store(shared, 0, prompt, batch)
+    again = store(shared, 0, prompt, batch)
+    fresh = store(DecodeCache(HostCacheModule(), max_tail=8), 0, prompt, batch)
+    assert again["per"] == fresh["per"] and again["splits"] == fresh["splits"]
+    assert np.array_equal(again["bounds_host"], fresh["bounds_host"])
+    assert np.array_equal(DecodeCache._task_items(again), DecodeCache._task_items(fresh))
+
+
+def test_layouts_are_bounded():
+    cache = DecodeCache(HostCacheModule(), max_tail=8)
+    cache.LAYOUTS = 3
+    for tiles in range(1, 7):
+        store(cache, 0, 64 * tiles)
+    assert len(cache.layouts) == 3
+    assert store(cache, 0, 64)["splits"] >= 1 and len(cache.layouts) == 3

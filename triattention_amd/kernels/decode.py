@@ -199,12 +199,17 @@ class _LayerStore:
         # tail base (tokens moved from the tail into the cache since the store)
         self.grow_tiles = 0
         self.tb = 0
+        self.tail_clear = False  # the tails and the tail base are zero and no step has run on them
         self.arrays["tail_base"] = torch.zeros(2, dtype=torch.int64, device=device)
 
-    def _regrow(self, name, shape, fill, dtype):
-        """Array ``name`` at ``shape``, filled with ``fill`` and holding the old contents in its corner."""
+    def _regrow(self, name, shape, fill, dtype, written=False):
+        """Array ``name`` at ``shape``, filled with ``fill`` and holding the old contents in its corner.
+        ``written``: the coming store writes every element of a new array (no fill)."""
         old = self.arrays[name]
         if old is not None and tuple(old.shape) == tuple(shape):
+            return
+        if old is None and written:
+            self.arrays[name] = torch.empty(shape, dtype=dtype, device=self.device)
             return
         new = torch.full(shape, fill, dtype=dtype, device=self.device) if fill is not None else \
             torch.zeros(shape, dtype=dtype, device=self.device)
@@ -222,23 +227,32 @@ class _LayerStore:
         relayout = cap_rows != self.cap["rows"] or maxn != self.maxn or tiles_max != self.tiles_max
         self.cap["rows"], self.maxn, self.tiles_max = cap_rows, maxn, tiles_max
         hk, i32, f32 = self.hk, torch.int32, torch.float32
+        # (the store writes its rows of the metadata, scales and statistics whole: with no row to spare
+        # they need no fill)
+        whole = not ragged and self.rows == 0
         if relayout:
             for name in ("entry", "kinfo", "slot"):
-                self._regrow(name, (cap_rows, hk, maxn), 0, i32)
-            self._regrow("count", (cap_rows, hk), 0, i32)
-            self._regrow("fmt", (cap_rows, tiles_max), 1, i32)
-            self._regrow("prompt", (cap_rows,), 0, i32)
-            self._regrow("ka", (cap_rows, hk, tiles_max, 4), 1.0, f32)
-            self._regrow("kstat", (cap_rows, hk, 3, 128), 0.0, f32)
-            self._regrow("vstat", (cap_rows, hk, 3, 128), 0.0, f32)
+                self._regrow(name, (cap_rows, hk, maxn), 0, i32, whole)
+            self._regrow("count", (cap_rows, hk), 0, i32, whole)
+            self._regrow("fmt", (cap_rows, tiles_max), 1, i32, whole)
+            self._regrow("prompt", (cap_rows,), 0, i32, whole)
+            self._regrow("ka", (cap_rows, hk, tiles_max, 4), 1.0, f32, whole)
+            self._regrow("kstat", (cap_rows, hk, 3, 128), 0.0, f32, whole)
+            self._regrow("vstat", (cap_rows, hk, 3, 128), 0.0, f32, whole)
+            tail = (cap_rows, hk, self.max_tail, 128)
+            if self.arrays["tail_k"] is None:
+                # (both in one allocation and one fill)
+                self.arrays["tail_k"], self.arrays["tail_v"] = torch.zeros((2,) + tail, dtype=torch.bfloat16,
+                                                                           device=self.device).unbind(0)
+                self.tail_clear = True
             for name in ("tail_k", "tail_v"):
-                self._regrow(name, (cap_rows, hk, self.max_tail, 128), 0.0, torch.bfloat16)
-            self._regrow("grow", (cap_rows, hk, 4), -1, i32)
-            self._regrow("count0", (cap_rows, hk), 0, i32)
+                self._regrow(name, tail, 0.0, torch.bfloat16)
+            self._regrow("grow", (cap_rows, hk, 4), -1, i32, whole and not self.grow_tiles)
+            self._regrow("count0", (cap_rows, hk), 0, i32, whole)
         if (int4 or self.arrays["ka4"] is not None) and (relayout or self.arrays["ka4"] is None):
-            self._regrow("ka4", (cap_rows, hk, tiles_max, 4), 1.0, f32)
+            self._regrow("ka4", (cap_rows, hk, tiles_max, 4), 1.0, f32, whole)
         if (exact or self.arrays["xslot"] is not None) and (relayout or self.arrays["xslot"] is None):
-            self._regrow("xslot", (cap_rows, hk), -1, i32)
+            self._regrow("xslot", (cap_rows, hk), -1, i32, whole)
         for kind, (words, dtype) in self.RECORD.items():
             # the decode op takes non-empty K8 / V8 / V4 arrays: at least one (zero) record each
             need = max(records[kind], 1 if kind != "k4" else 0)
@@ -246,13 +260,15 @@ class _LayerStore:
                 continue
             cap = grow(max(need, 1), self.cap[kind])
             if cap != self.cap[kind] or self.arrays[kind] is None:
-                self._regrow(kind, (cap, words), None, dtype)
+                # (the store writes every record that it keeps; a placeholder and growth room stay zero)
+                self._regrow(kind, (cap, words), None, dtype, whole and cap == records[kind] and not self.grow_tiles)
                 self.cap[kind] = cap
         if exact or self.arrays["kx"] is not None:
             cap = grow(max(records["x"], 1), self.cap["x"])
             if cap != self.cap["x"] or self.arrays["kx"] is None:
-                self._regrow("kx", (cap * KX_BYTES,), None, torch.uint8)
-                self._regrow("vx", (cap * KX_BYTES,), None, torch.uint8)
+                full = whole and exact and cap == records["x"] and not self.grow_tiles
+                self._regrow("kx", (cap * KX_BYTES,), None, torch.uint8, full)
+                self._regrow("vx", (cap * KX_BYTES,), None, torch.uint8, full)
                 self.cap["x"] = cap
 
 
@@ -263,6 +279,8 @@ class DecodeCache:
         self.ragged = False
         self.out_dtype = None
         self.meta_cache = {}
+        self.layouts = {}
+        self._cus = None
         self.wave = None
         # None: the balanced split partition; an int: the reference's uniform split of `per` tiles
         self.per = None
@@ -315,8 +333,7 @@ class DecodeCache:
         kind, info = growth_kinds(bands, hk, exact_kv) if G else (np.zeros(hk, np.int64), np.full(hk, -1, np.int32))
         nx = len(exact_kv)
         xstride = tiles + G
-        seq = dict(k8=int(meta["is8"].sum()), k4=int(meta["is4"].sum()), v8=int(meta["vsel"][I8].sum()),
-                   v4=int(meta["vsel"][I4].sum()), x=nx * xstride)
+        seq = dict(meta["records"], x=nx * xstride)
         # growth room per sequence: G records per KV head of each kind (V always INT8)
         room = dict(k8=int((kind == 8).sum()) * G, k4=int((kind == 4).sum()) * G,
                     v8=int(((kind == 8) | (kind == 4)).sum()) * G, v4=0, x=0)
@@ -356,9 +373,11 @@ class DecodeCache:
         self.step.zero_()
         self.host_step = 0
         st.tb = 0
-        a["tail_base"].zero_()
-        a["tail_k"][:st.rows].zero_()
-        a["tail_v"][:st.rows].zero_()
+        if not (st.tail_clear and row0 == 0):
+            a["tail_base"].zero_()
+            a["tail_k"][:st.rows].zero_()
+            a["tail_v"][:st.rows].zero_()
+        st.tail_clear = False
         self.layers[layer] = self._assemble(st)
 
     def _metadata(self, bands, tiles, hk, codes, exact_kv, device):
@@ -371,6 +390,9 @@ class DecodeCache:
         hit = self.meta_cache.get(key)
         if hit is None:
             meta = sequence_metadata(b, tiles, hk, codes, exact_kv)
+            meta["records"] = dict(k8=int(meta["is8"].sum()), k4=int(meta["is4"].sum()),
+                                   v8=int(meta["vsel"][I8].sum()), v4=int(meta["vsel"][I4].sum()))
+            meta["kept"], meta["key"] = int(meta["count"].sum()), key
             flags = torch.full((hk,), -1, dtype=torch.int32)
             for xs, h in enumerate(exact_kv):
                 flags[h] = xs
@@ -378,15 +400,31 @@ class DecodeCache:
             hit = self.meta_cache[key] = (meta, dev)
         return hit
 
-    def _assemble(self, st):
-        """The layer entry the decode op reads: views of the store's arrays over its sequences, and the
-        split partition over every stored group (host metadata, no device sync)."""
-        groups, device = st.groups, st.device
-        a, rows = st.arrays, st.rows
+    LAYOUTS = 64  # split partitions kept (one per shape of a one-group cache)
+
+    def _layout(self, st):
+        """The split partition over every stored group (host metadata, no device sync): per, splits, bounds on
+        the host and the device, and room for the task items that ``plan`` derives from them.  It depends on
+        lengths, bands and the wave alone, so every prompt of one shape (each layer of a model, each new
+        prompt) shares it; ragged batches of several stores compute their own."""
         if self.wave is None:
             cus = self.module.device_cus() if hasattr(self.module, "device_cus") else \
-                torch.cuda.get_device_properties(device).multi_processor_count
+                torch.cuda.get_device_properties(st.device).multi_processor_count
             self.wave = cus * max(1, min(self.module.decode_occupancy(), SPLITS_PER_CU))
+        if len(st.groups) > 1:
+            return self._partition(st)
+        g = st.groups[0]
+        key = (g["meta"]["key"], g["batch"], st.maxn, st.grow_tiles, self.per, self.wave)
+        hit = self.layouts.pop(key, None)
+        if hit is None:
+            hit = self._partition(st)
+        self.layouts[key] = hit  # most recently used last
+        while len(self.layouts) > self.LAYOUTS:
+            self.layouts.pop(next(iter(self.layouts)))
+        return hit
+
+    def _partition(self, st):
+        groups, device, rows = st.groups, st.device, st.rows
         # Split partition, from the host metadata (no device sync).
         # - Up to BALANCE_TILES kept tiles per slot (one wave of SPLITS_PER_CU workgroups per CU;
         #   C1: 16384 tiles on 1024 slots): every SIMD runs one split, so the kernel lasts as
@@ -399,7 +437,7 @@ class DecodeCache:
         #   102.1 us at 28 tiles per split, 103.2 at 30, 104.4 at 32, 105.2 at 26, 106.7 at 24,
         #   108.2 at 36; balanced over 4096-8192 slots 138-168 us in an earlier build).
         # - self.per set: always runs of that many tiles.  At most 64 tiles per split.
-        kept = sum(g["batch"] * int(g["meta"]["count"].sum()) for g in groups)
+        kept = sum(g["batch"] * g["meta"]["kept"] for g in groups)
         if self.per is None and kept <= BALANCE_TILES * self.wave:
             parts, splits = balanced_partition([g["meta"] for g in groups], [g["batch"] for g in groups], self.wave)
             bounds_host = torch.cat([p[None].expand(g["batch"], -1, -1) for p, g in zip(parts, groups)])
@@ -425,10 +463,19 @@ class DecodeCache:
             splits = bounds_host.shape[2] - 1
             per = int(bounds_host.diff(dim=2).max())
             bounds = bounds_host.to(device)
+        return dict(per=per, splits=splits, bounds=bounds,
+                    bounds_host=None if bounds_host is None else bounds_host.numpy())
+
+    def _assemble(self, st):
+        """The layer entry the decode op reads: views of the store's arrays over its sequences, and the
+        split partition."""
+        groups, a, rows = st.groups, st.arrays, st.rows
+        layout = self._layout(st)
         some = lambda name, n: a[name][:max(1, n)]
         has_x = any(g["exact"] for g in groups)
-        return dict(groups=groups, store=st, prompt=a["prompt"][:rows], maxn=st.maxn, per=per, splits=splits,
-                    bounds=bounds, bounds_host=None if bounds_host is None else bounds_host.numpy(),
+        return dict(groups=groups, store=st, prompt=a["prompt"][:rows], maxn=st.maxn, per=layout["per"],
+                    splits=layout["splits"], bounds=layout["bounds"], bounds_host=layout["bounds_host"], layout=layout,
+                    calls={},
                     fmt=a["fmt"][:rows], slot=a["slot"][:rows], entry=a["entry"][:rows], kinfo=a["kinfo"][:rows],
                     count=a["count"][:rows], k8=some("k8", st.n["k8"]),
                     k4=some("k4", st.n["k4"]) if a["k4"] is not None else None, ka=a["ka"][:rows],
@@ -460,10 +507,22 @@ class DecodeCache:
         st = e["store"]
         dtype = self.out_dtype or q.dtype
         out = torch.empty(q.shape, dtype=dtype, device=q.device)
-        plan = self.plan(layer, q, k, out, scale)
+        # the plan by the raw shapes and strides of this call's tensors (``out`` is contiguous): ``plan`` and
+        # ``run`` compare geometries dimension by dimension, which a step of the same shapes need not repeat
+        shapes = (q.shape, q.stride(), q.dtype, q.device, dtype, k.shape, k.stride(), k.dtype, k.device, scale)
+        plan = e["calls"].get(shapes)
+        same = v.shape == k.shape and v.stride() == k.stride() and v.dtype == k.dtype and v.device == k.device
+        checked = plan is not None and same
+        if plan is None:
+            plan = self.plan(layer, q, k, out, scale)
         if st.grow_tiles:
             self._spill_plan(e).run()
-        plan.run(q, k, v, out, short_tail=self.short_tail(layer, q.shape[1]))
+        short = self.short_tail(layer, q.shape[1])
+        if checked:
+            plan.launch(q, k, v, out, short_tail=short)
+        else:
+            plan.run(q, k, v, out, short_tail=short)
+            e["calls"][shapes] = plan
         return out
 
     # the merge runs as one wave per (sequence, q-head) while the tail holds at most SHORT_TAIL tokens on a
@@ -489,7 +548,9 @@ class DecodeCache:
         itself at every replay (a captured one-wave launch would keep that form at later, longer tails)."""
         if self.capturing:
             return False
-        if self.layers[layer]["batch"] * hq < self.SHORT_WIDE * self.module.device_cus():
+        if self._cus is None:
+            self._cus = self.module.device_cus()
+        if self.layers[layer]["batch"] * hq < self.SHORT_WIDE * self._cus:
             return False
         return self.tail_tokens(layer) <= self.SHORT_TAIL
 
@@ -507,8 +568,11 @@ class DecodeCache:
         if key not in e:
             hq = q.shape[1]
             if self.tasks and e["xslot"] is None and "tasks" not in e and hasattr(self.module, "decode_tasks"):
-                items_host = self._task_items(e)
-                items = torch.from_numpy(items_host).to(q.device)
+                layout = e["layout"]
+                if "items" not in layout:
+                    items_host = self._task_items(e)
+                    layout["items"] = items_host, torch.from_numpy(items_host).to(q.device)
+                items_host, items = layout["items"]
                 e["tasks"] = self.module.decode_tasks(e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"],
                                                       e["slot"], e["per"], e["bounds"], items)
                 if e["grow_splits"]:

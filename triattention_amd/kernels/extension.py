@@ -36,9 +36,9 @@ D = 128
 STAT_BLOCKS = 64
 K8_WORDS, K4_WORDS, V16_WORDS, V8_WORDS, V4_WORDS = 2048, 1024, 4096, 2048, 1024
 
-EXPORTS = ("tri_last_error", "tri_prepare_qk", "tri_pack_v", "tri_prepare", "tri_attention", "tri_pack_exact", "tri_decode",
-           "tri_decode_partials", "tri_decode_merge", "tri_decode_short_tail", "tri_decode_merge_short_tail",
-           "tri_decode_partials_timed", "tri_decode_noalloc",
+EXPORTS = ("tri_last_error", "tri_prepare_qk", "tri_pack_v", "tri_prepare", "tri_attention", "tri_pack_exact",
+           "tri_decode", "tri_decode_partials", "tri_decode_merge", "tri_decode_short_tail",
+           "tri_decode_merge_short_tail", "tri_decode_partials_timed", "tri_decode_noalloc",
            "tri_decode_tasks", "tri_cache_store", "tri_tail_spill", "tri_decode_occupancy", "tri_device_cus",
            "tri_stream_read", "tri_issue_probe", "tri_prefill_pairs")
 KX_BYTES = 16384
@@ -127,6 +127,16 @@ class Module:
     def _stream(device) -> int:
         return torch.cuda.current_stream(device).cuda_stream
 
+    def _launch(self, device, fn, *args):
+        """``fn(*args, stream)`` on ``device``'s current stream, with that device current."""
+        index = device.index if device.index is not None else torch.cuda.current_device()
+        stream = torch.cuda.current_stream(index).cuda_stream
+        if torch.cuda.current_device() == index:
+            self._call(fn, *args, stream)
+        else:
+            with torch.cuda.device(index):
+                self._call(fn, *args, stream)
+
     # -------------------------------------------------------------- prepare_qk
     @staticmethod
     def _check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x):
@@ -180,10 +190,9 @@ class Module:
         Extension: ``k4x`` (uint32, as many words as ``kp``, with the INT4 buffers) receives the K4 records
         expanded to 16 * code bytes in the K8 layout, which ``attention(..., k4x=...)`` reads."""
         b, hq, hk, t = self._check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x)
-        with torch.cuda.device(q.device):
-            self._call(self.lib.tri_prepare_qk, _ptr(q), q.stride(0), q.stride(1), q.stride(2), _ptr(k), k.stride(0),
-                       k.stride(1), k.stride(2), b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka), _ptr(partial),
-                       _ptr(kstat), _ptr(q4), _ptr(qa4), _ptr(k4p), _ptr(ka4), _ptr(k4x), self._stream(q.device))
+        self._launch(q.device, self.lib.tri_prepare_qk, _ptr(q), q.stride(0), q.stride(1), q.stride(2), _ptr(k),
+                     k.stride(0), k.stride(1), k.stride(2), b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka),
+                     _ptr(partial), _ptr(kstat), _ptr(q4), _ptr(qa4), _ptr(k4p), _ptr(ka4), _ptr(k4x))
 
     # ------------------------------------------------------------------ pack_v
     def pack_v(self, v, partial, vstat, v16p=None, v8p=None, v4p=None, v8sum=None):
@@ -192,9 +201,8 @@ class Module:
         Extension: ``v8sum`` (int32 [B*Hkv*tiles*128], with ``v8p``) receives -127 times each channel's
         sum of each tile's V8 codes, which ``attention(..., v8sum=...)`` starts its P V products from."""
         b, hk, t = self._check_v(v, partial, vstat, v16p, v8p, v4p, v8sum)
-        with torch.cuda.device(v.device):
-            self._call(self.lib.tri_pack_v, _ptr(v), v.stride(0), v.stride(1), v.stride(2), b, hk, t, _ptr(partial),
-                       _ptr(vstat), _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum), self._stream(v.device))
+        self._launch(v.device, self.lib.tri_pack_v, _ptr(v), v.stride(0), v.stride(1), v.stride(2), b, hk, t,
+                     _ptr(partial), _ptr(vstat), _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum))
 
     # ----------------------------------------------------------------- prepare
     def prepare(self, q, k, v, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x, vpartial, vstat, v16p, v8p,
@@ -206,16 +214,14 @@ class Module:
         _check(self._check_v(v, vpartial, vstat, v16p, v8p, v4p, v8sum) == (b, hk, t), "V [B,Hkv,T,128] like K")
         if exact is not None:
             _check(self._check_exact(k, v, exact, nx, kx, vx)[1] == hq, "exact flags [Hq]")
-        with torch.cuda.device(q.device):
-            self._call(self.lib.tri_prepare, _ptr(q), *q.stride()[:3], _ptr(k), *k.stride()[:3], _ptr(v),
-                       *v.stride()[:3], b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka), _ptr(kpartial),
-                       _ptr(kstat), _ptr(q4), _ptr(qa4), _ptr(k4p), _ptr(ka4), _ptr(k4x), _ptr(vpartial), _ptr(vstat),
-                       _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum), _ptr(exact), int(nx), _ptr(kx), _ptr(vx),
-                       self._stream(q.device))
+        self._launch(q.device, self.lib.tri_prepare, _ptr(q), *q.stride()[:3], _ptr(k), *k.stride()[:3], _ptr(v),
+                     *v.stride()[:3], b, hq, hk, t, _ptr(q8), _ptr(qa), _ptr(kp), _ptr(ka), _ptr(kpartial),
+                     _ptr(kstat), _ptr(q4), _ptr(qa4), _ptr(k4p), _ptr(ka4), _ptr(k4x), _ptr(vpartial), _ptr(vstat),
+                     _ptr(v16p), _ptr(v8p), _ptr(v4p), _ptr(v8sum), _ptr(exact), int(nx), _ptr(kx), _ptr(vx))
 
     # --------------------------------------------------------------- attention
     def attention(self, order, bands, groups, entries, v16p, v8p, v4p, vstat, q8, k8p, qa8, ka8, q4, k4p, qa4, ka4,
-                  out, scale, exact=None, q=None, kx=None, vx=None, nx=0, v8sum=None, k4x=None):
+                  out, scale, exact=None, q=None, kx=None, vx=None, nx=0, v8sum=None, k4x=None, f16_only=False):
         """Banded causal attention: per key tile skip / INT8 QK x FP16 or INT8 PV / INT4 QK x INT8 PV.
 
         Extension: ``exact`` (int32 [Hq] on the device, 0 or 1 + record slot
@@ -223,7 +229,9 @@ class Module:
         ``kx``/``vx`` records of ``pack_exact`` computes the flagged q-heads as
         exact causal attention on the unquantized operands.  ``v8sum``: what
         ``pack_v(..., v8sum=...)`` wrote for ``v8p`` (the same result, fewer MFMAs).  ``k4x``: what
-        ``prepare_qk(..., k4x=...)`` wrote for ``k4p`` (the same result, fewer VALU instructions)."""
+        ``prepare_qk(..., k4x=...)`` wrote for ``k4p`` (the same result, fewer VALU instructions).
+        ``f16_only``: the caller knows that no band has INT8 or INT4 key tiles (a call without V8
+        records otherwise copies ``bands`` to the host to check that)."""
         _check(q8.dtype == torch.int8 and q8.dim() == 4 and q8.size(3) == D and q8.is_contiguous(), "Q8 [B,Hq,T,128]")
         b, h, t, _ = q8.shape
         hk = vstat.numel() // (b * 3 * D)
@@ -236,7 +244,8 @@ class Module:
                "bands [Hq,2] or task tables")
         _check((q4 is None) == (k4p is None) == (qa4 is None) == (ka4 is None), "INT4 Q/K operands (all or none)")
         _check(v16p is not None and v16p.numel() == b * hk * tiles * V16_WORDS, "packed V16")
-        _check(v8p is not None or (q4 is None and _only_f16(bands, tiles)), "packed V8 required by INT8/INT4 bands")
+        _check(v8p is not None or (q4 is None and (f16_only or _only_f16(bands, tiles))),
+               "packed V8 required by INT8/INT4 bands")
         _check(out.dim() == 4 and tuple(out.shape) == (b, h, t, D) and out.stride(3) == 1 and
                out.dtype in (torch.float32, torch.bfloat16, torch.float16), "output [B,Hq,T,128]")
         dt = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[out.dtype]
@@ -251,21 +260,19 @@ class Module:
         _check(k4x is None or (q4 is not None and k4x.dtype == torch.uint32 and k4x.is_contiguous() and
                                k4x.numel() == b * hk * tiles * K8_WORDS), "expanded K4 records (with the INT4 operands)")
         qs = q.stride() if exact is not None else (0, 0, 0)
-        with torch.cuda.device(q8.device):
-            self._call(self.lib.tri_attention, _ptr(order), order.numel(), _ptr(bands), b, h, hk, t, _ptr(v16p),
-                       _ptr(v8p), _ptr(vstat), _ptr(q8), _ptr(k8p), _ptr(qa8), _ptr(ka8), _ptr(q4), _ptr(k4p),
-                       _ptr(qa4), _ptr(ka4), _ptr(out), dt, out.stride(0), out.stride(1), out.stride(2),
-                       float(scale), _ptr(exact), _ptr(q if exact is not None else None), qs[0], qs[1], qs[2],
-                       _ptr(kx if exact is not None else None), _ptr(vx if exact is not None else None),
-                       int(nx) if exact is not None else 0, _ptr(v8sum), _ptr(k4x), self._stream(q8.device))
+        self._launch(q8.device, self.lib.tri_attention, _ptr(order), order.numel(), _ptr(bands), b, h, hk, t,
+                     _ptr(v16p), _ptr(v8p), _ptr(vstat), _ptr(q8), _ptr(k8p), _ptr(qa8), _ptr(ka8), _ptr(q4),
+                     _ptr(k4p), _ptr(qa4), _ptr(ka4), _ptr(out), dt, out.stride(0), out.stride(1), out.stride(2),
+                     float(scale), _ptr(exact), _ptr(q if exact is not None else None), qs[0], qs[1], qs[2],
+                     _ptr(kx if exact is not None else None), _ptr(vx if exact is not None else None),
+                     int(nx) if exact is not None else 0, _ptr(v8sum), _ptr(k4x))
         return out
 
     def pack_exact(self, k, v, exact, nx, kx, vx):
         """bf16 K/V of the exact KV heads -> KX/VX records [B][nx][tiles] (16 KiB each; extension)."""
         b, h, hk, t = self._check_exact(k, v, exact, nx, kx, vx)
-        with torch.cuda.device(k.device):
-            self._call(self.lib.tri_pack_exact, _ptr(k), *k.stride()[:3], _ptr(v), *v.stride()[:3], b, h, hk, t,
-                       _ptr(exact), int(nx), _ptr(kx), _ptr(vx), self._stream(k.device))
+        self._launch(k.device, self.lib.tri_pack_exact, _ptr(k), *k.stride()[:3], _ptr(v), *v.stride()[:3], b, h, hk,
+                     t, _ptr(exact), int(nx), _ptr(kx), _ptr(vx))
 
     # ------------------------------------------------------------------ decode
     def decode(self, q, k8c, k4c, ka, ka4, entry, kinfo, count, fmt, slot, v8, v4, vstat, kstat, ktail, vtail, kcur,
@@ -408,11 +415,9 @@ class Module:
         _check(items is None or (items.dtype == torch.int32 and items.is_cuda and 1 <= n <= b * hk * splits),
                "decode_tasks: items int32 on the device, at most one per split")
         table = torch.empty(n * TASK_WORDS, dtype=torch.int32, device=entry.device)
-        with torch.cuda.device(entry.device):
-            self._call(self.lib.tri_decode_tasks, _ptr(ka), _ptr(ka4), _ptr(entry), _ptr(kinfo), _ptr(count),
-                       _ptr(fmt), _ptr(slot), b, hk, maxn, int(per), tiles_max, _ptr(bounds),
-                       splits if bounds is not None else 0, _ptr(items), n if items is not None else 0, _ptr(table),
-                       self._stream(entry.device))
+        self._launch(entry.device, self.lib.tri_decode_tasks, _ptr(ka), _ptr(ka4), _ptr(entry), _ptr(kinfo),
+                     _ptr(count), _ptr(fmt), _ptr(slot), b, hk, maxn, int(per), tiles_max, _ptr(bounds),
+                     splits if bounds is not None else 0, _ptr(items), n if items is not None else 0, _ptr(table))
         return table, n
 
     def cache_store(self, bands, exact, t, kp, k4p, ka, ka4, kstat, vstat, v8p, v4p, kx, vx, nx, row0, dst, used,
@@ -458,15 +463,13 @@ class Module:
                    f"cache_store: {kind} record array")
         _check(dst["kx"] is None or dst["kx"].numel() >= cap["x"] * KX_BYTES, "cache_store: KX/VX record arrays")
         p = _ptr
-        with torch.cuda.device(vstat.device):
-            self._call(self.lib.tri_cache_store, p(bands), p(exact), b, hq, hk, int(t), int(nx), xstride, p(kp), p(k4p),
-                       p(ka),
-                       p(ka4), p(kstat), p(vstat), p(v8p), p(v4p), p(kx), p(vx), int(row0), rows, maxn, tiles_max,
-                       p(dst["entry"]), p(dst["kinfo"]), p(dst["slot"]), p(dst["count"]), p(dst["fmt"]),
-                       p(dst["prompt"]), p(dst["xslot"]), p(dst["ka"]), p(dst["ka4"]), p(dst["kstat"]),
-                       p(dst["vstat"]), p(dst["k8"]), used["k8"], cap["k8"], p(dst["k4"]), used["k4"], cap["k4"],
-                       p(dst["v8"]), used["v8"], cap["v8"], p(dst["v4"]), used["v4"], cap["v4"], p(dst["kx"]),
-                       p(dst["vx"]), used["x"], cap["x"], self._stream(vstat.device))
+        self._launch(vstat.device, self.lib.tri_cache_store, p(bands), p(exact), b, hq, hk, int(t), int(nx), xstride,
+                     p(kp), p(k4p), p(ka), p(ka4), p(kstat), p(vstat), p(v8p), p(v4p), p(kx), p(vx), int(row0), rows,
+                     maxn, tiles_max, p(dst["entry"]), p(dst["kinfo"]), p(dst["slot"]), p(dst["count"]),
+                     p(dst["fmt"]), p(dst["prompt"]), p(dst["xslot"]), p(dst["ka"]), p(dst["ka4"]), p(dst["kstat"]),
+                     p(dst["vstat"]), p(dst["k8"]), used["k8"], cap["k8"], p(dst["k4"]), used["k4"], cap["k4"],
+                     p(dst["v8"]), used["v8"], cap["v8"], p(dst["v4"]), used["v4"], cap["v4"], p(dst["kx"]),
+                     p(dst["vx"]), used["x"], cap["x"])
 
     def plan_tail_spill(self, step, tail_base, ktail, vtail, grow, cap, prompt, dst, tasks=None):
         """Validate and marshal one layer's ``tail_spill`` launch (extension; the reference clamps its
@@ -575,6 +578,10 @@ class DecodePlan:
         if _geometry(q) != self.qgeom or _geometry(kcur) != self.cgeom or _geometry(vcur) != self.cgeom or \
                 _geometry(out) != self.ogeom:
             raise RuntimeError("decode plan: q / k / v / out differ in shape, strides, dtype or device from the plan")
+        return self.launch(q, kcur, vcur, out, phase, events, short_tail)
+
+    def launch(self, q, kcur, vcur, out, phase=3, events=None, short_tail=False):
+        """``run`` on tensors whose geometries are known to be the plan's."""
         a = self.args
         a[self.Q], a[self.KC], a[self.VC], a[self.OUT] = q.data_ptr(), kcur.data_ptr(), vcur.data_ptr(), out.data_ptr()
         index = self.device.index if self.device.index is not None else torch.cuda.current_device()

@@ -225,7 +225,8 @@ class Prefill:
             extra = {} if exact is None else dict(exact=exact, q=q, kx=kx, vx=vx, nx=nx)
             self.module.attention(table.order, table.bands, None, None, packed[F16], packed[I8], packed[I4],
                                   ops["vstat"], ops["q8"], ops["kp"], ops["qa"], ops["ka"], ops["q4"], ops["k4"],
-                                  ops["qa4"], ops["ka4"], out, scale, v8sum=v8sum, k4x=k4x, **extra)
+                                  ops["qa4"], ops["ka4"], out, scale, v8sum=v8sum, k4x=k4x,
+                                  f16_only=table.formats == {F16}, **extra)
         if decode is not None:
             exact_kv = sorted(set(int(h) for h in self.bands_fn.bf16(layer))) if exact is not None else []
             self.decode_cache.store(layer, t, ops["kp"], ops["ka"], ops["kstat"], ops["vstat"], packed, decode[0],
