@@ -787,7 +787,8 @@ int tri_cache_store(const int32_t* bands, const int32_t* exact, int batch, int h
   a.capv8 = capv8;
   a.capv4 = capv4;
   a.capx = exact ? capx : 0;
-  const dim3 grid((tiles + tri::STORE_CHUNK - 1) / tri::STORE_CHUNK, hk, batch);
+  a.chunk = (int)std::min<int64_t>(tri::STORE_CHUNK, ((int64_t)tiles * hk * batch + tri::STORE_WGS - 1) / tri::STORE_WGS);
+  const dim3 grid((tiles + a.chunk - 1) / a.chunk, hk, batch);
   tri::cache_store_kernel<<<grid, tri::STORE_THREADS, 0, static_cast<hipStream_t>(stream)>>>(a);
   return check_launch("cache_store");
 }

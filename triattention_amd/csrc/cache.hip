@@ -14,23 +14,30 @@
 // Extension: KV heads kept exact (bf16) keep every tile with every q-head's bit set, select no quantized
 // record, and copy their KX / VX records whole.
 //
-// One workgroup per (tile chunk, KV head, sequence).  Every workgroup classifies the tiles of every KV
-// head of its sequence (a few thousand state evaluations) and scans them, so it knows each of its tiles'
-// entry index and record slots without any other workgroup; the chunk-0 workgroup of a head writes the
-// head's metadata row, and every workgroup copies the records of its chunk's kept tiles with coalesced
-// 16-byte accesses.
+// Every state depends on the tile's distance from the end alone, so each head's kept, INT8-K, INT4-K, INT8-V
+// and INT4-V tiles are tile 0 and runs of consecutive tiles whose ends follow from the largest w8 and w4 of
+// the group: entry indices and record slots have closed forms, and no workgroup scans tiles or waits for
+// another.  One workgroup per (run of tiles, KV head, sequence): it forms every head's counts (one thread
+// per head), copies its tiles' records with 16-byte accesses, K and V loads in flight together, and the
+// chunk-0 workgroup of a head writes the head's metadata row.  HBM-bound for many tiles, one launch's latency
+// for few: against classifying and scanning every head's tiles in every workgroup and 16 tiles copied one
+// after another, 64 tiles x 4 KV heads (one exact) 43.5 -> 10.3 us, one tile x 8 KV heads 12.0 -> 7.3 us,
+// 64 tiles x 8 KV heads x 32 sequences 92 -> 94 us.
 #include "common.h"
 
 namespace tri {
 
-constexpr int STORE_CHUNK = 16;    // tiles whose records one workgroup copies
+// Tiles whose records one workgroup copies: as many as keep the launch at STORE_WGS workgroups, at most
+// STORE_CHUNK (few tiles: one each, so that their latencies overlap; many: each workgroup's counts are shared by
+// more copies.  At most 2 / 4 / 8 per workgroup: 256 tiles 12.6 / 17.8 / - (one: 10.1), 16,384 tiles 113 / 94 / 110 us).
+constexpr int STORE_CHUNK = 4, STORE_WGS = 2048;
 constexpr int STORE_THREADS = 256;
 constexpr int STORE_MAX_HQ = 256;  // q-heads whose bands the kernel stages in LDS
 
 struct CacheStoreArgs {
   const int32_t* bands;  // [hq][2] (w8, w4)
   const int32_t* exact;  // [hk]: -1 for a quantized KV head, else its slot among the exact heads; may be null
-  int hq, hk, t, tiles, nx, batch;
+  int hq, hk, t, tiles, nx, batch, chunk;  // chunk: tiles per workgroup
   int xstride;  // records per (sequence, exact head) in the destination (>= tiles: room for tail tiles)
   // sources: the Prefill call's outputs, [batch][hk][tiles] records and scales
   const uint8_t* kp;   // K8
@@ -66,200 +73,137 @@ struct CacheStoreArgs {
   int64_t cap8, cap4, capv8, capv4, capx;
 };
 
-// counts of one tile packed in 12-bit fields: kept | INT4 K << 12 | INT8 K << 24 | INT8 V << 36 | INT4 V << 48
-__device__ __forceinline__ uint64_t tile_counts(bool kept, bool is4, bool is8, bool v8, bool v4) {
-  return (uint64_t)kept | (uint64_t)is4 << 12 | (uint64_t)is8 << 24 | (uint64_t)v8 << 36 | (uint64_t)v4 << 48;
-}
-__device__ __forceinline__ int field(uint64_t c, int f) { return (int)((c >> (12 * f)) & 0xfffu); }
-
-struct TileClass {
-  bool kept, is4, is8, v8, v4;
-  int mask;
+// A head's tile runs: kept tiles are 0 and [keep, tiles), INT8-K ones (quantized heads) 0 and [k8, tiles),
+// INT4-K ones [keep, k8), INT8-V ones 0 and [v8, tiles), INT4-V ones [keep, v8).
+struct HeadRuns {
+  int keep, k8, v8;
 };
-
-__device__ __forceinline__ TileClass classify(const int* sb, int g, bool ex, int tiles, int j) {
-  TileClass c;
-  int kv = 0, mask = 0;
-  const int d = tiles - 1 - j;
-#pragma unroll 1
+__device__ __forceinline__ HeadRuns head_runs(const int* bands, int g, bool ex, int tiles) {
+  int w8 = 0, w4 = 0;
   for (int r = 0; r < g; ++r) {
-    const int w8 = sb[2 * r], w4 = sb[2 * r + 1];
-    const int s = ex ? 8 : (j == 0 || d < w8) ? 8 : (d < w4 ? 4 : 0);
-    kv = max(kv, s);
-    mask |= (s > 0 ? 1 : 0) << r;
+    w8 = max(w8, bands[2 * r]);
+    w4 = max(w4, bands[2 * r + 1]);
   }
-  const bool vi8 = j == 0 || d < NEAR_V8;
-  c.kept = kv > 0;
-  c.is4 = !ex && kv == 4;
-  c.is8 = !ex && kv == 8;
-  c.v8 = !ex && c.kept && vi8;
-  c.v4 = !ex && c.kept && !vi8;
-  c.mask = mask;
-  return c;
+  HeadRuns h;
+  h.keep = ex ? min(1, tiles) : max(1, tiles - max(w8, w4));
+  h.k8 = max(1, tiles - w8);
+  h.v8 = max(h.keep, tiles - NEAR_V8);
+  return h;
 }
-
-// exclusive prefix (this thread's) and total of v over the workgroup, in thread order
-__device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t& total, uint64_t* lds) {
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  uint64_t inc = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint64_t o = __shfl_up(inc, off, 64);
-    if (lane >= off) inc += o;
-  }
-  if (lane == 63) lds[w] = inc;
-  __syncthreads();
-  uint64_t before = 0;
-  total = 0;
-#pragma unroll
-  for (int i = 0; i < STORE_THREADS / 64; ++i) {
-    if (i < w) before += lds[i];
-    total += lds[i];
-  }
-  __syncthreads();
-  return before + inc - v;
-}
-
-struct CopyDesc {
-  int64_t ksrc, kdst, vsrc, vdst;  // record indices (-1: nothing to copy)
-  int kbytes, vbytes;
-  int kind;  // 0 quantized K and V, 1 exact KX and VX
-};
 
 __global__ __launch_bounds__(STORE_THREADS) void cache_store_kernel(CacheStoreArgs a) {
   __shared__ int sb[2 * STORE_MAX_HQ];
-  __shared__ uint64_t scan_lds[STORE_THREADS / 64];
-  __shared__ CopyDesc desc[STORE_CHUNK];
+  __shared__ int4 sc[STORE_MAX_HQ];  // per KV head: INT4-K, INT8-K, INT8-V and INT4-V tiles
   const int tid = threadIdx.x;
   const int chunk = blockIdx.x, kh = blockIdx.y, s = blockIdx.z;
   const int g = a.hq / a.hk, tiles = a.tiles, row = a.row0 + s;
   for (int i = tid; i < 2 * a.hq; i += STORE_THREADS) sb[i] = a.bands[i];
-  if (tid < STORE_CHUNK) desc[tid] = CopyDesc{0, 0, 0, 0, 0, 0, 0};
   __syncthreads();
-  // this thread's run of tiles: [j0, j1)
-  const int run = (tiles + STORE_THREADS - 1) / STORE_THREADS;
-  const int j0 = min(tiles, tid * run), j1 = min(tiles, j0 + run);
-  // counts of the heads before kh (record numbering is (KV head, entry) order within a sequence), the
-  // sequence's totals (plain ints: summed over heads they outgrow the 12-bit packed fields), and this
-  // thread's prefix within head kh
-  int before_head[5] = {0, 0, 0, 0, 0}, seq_total[5] = {0, 0, 0, 0, 0};
-  uint64_t my_prefix = 0, head_total = 0;
+  for (int h = tid; h < a.hk; h += STORE_THREADS) {
+    int4 c = make_int4(0, 0, 0, 0);
+    if (a.exact == nullptr || a.exact[h] < 0) {
+      const HeadRuns r = head_runs(sb + 2 * h * g, g, false, tiles);
+      c = make_int4(r.k8 - r.keep, 1 + tiles - r.k8, 1 + tiles - r.v8, r.v8 - r.keep);
+    }
+    sc[h] = c;
+  }
+  __syncthreads();
+  // record numbering is (KV head, entry) order within a sequence: the counts of the heads before kh, and the
+  // sequence's totals
+  int4 before = make_int4(0, 0, 0, 0), total = before;
   for (int h = 0; h < a.hk; ++h) {
-    const bool ex = a.exact != nullptr && a.exact[h] >= 0;
-    uint64_t mine = 0;
-    for (int j = j0; j < j1; ++j) {
-      const TileClass c = classify(sb + 2 * h * g, g, ex, tiles, j);
-      mine += tile_counts(c.kept, c.is4, c.is8, c.v8, c.v4);
-    }
-    uint64_t total;
-    const uint64_t pre = block_scan(mine, total, scan_lds);
-    if (h == kh) {
-      my_prefix = pre;
-      head_total = total;
-    }
-#pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      if (h < kh) before_head[f] += field(total, f);
-      seq_total[f] += field(total, f);
-    }
+    const int4 c = sc[h];
+    if (h == kh) before = total;
+    total = make_int4(total.x + c.x, total.y + c.y, total.z + c.z, total.w + c.w);
   }
   const bool ex = a.exact != nullptr && a.exact[kh] >= 0;
   const int xs = ex ? a.exact[kh] : 0;
+  const HeadRuns runs = head_runs(sb + 2 * kh * g, g, ex, tiles);
+  const int64_t base4 = a.o4 + (int64_t)s * total.x + before.x, base8 = a.o8 + (int64_t)s * total.y + before.y;
+  const int64_t basev8 = a.ov8 + (int64_t)s * total.z + before.z, basev4 = a.ov4 + (int64_t)s * total.w + before.w;
+  // K and V record slots of kept tile j of this (quantized) head
+  auto is4 = [&](int j) { return !ex && j > 0 && j < runs.k8; };
+  auto v8 = [&](int j) { return j == 0 || j >= runs.v8; };
+  auto kslot = [&](int j) { return is4(j) ? base4 + (j - runs.keep) : base8 + (j == 0 ? 0 : 1 + (j - runs.k8)); };
+  auto vslot = [&](int j) { return !v8(j) ? basev4 + (j - runs.keep) : basev8 + (j == 0 ? 0 : 1 + (j - runs.v8)); };
   const int64_t hb_src = (int64_t)s * a.hk + kh;
   const int64_t hb = (int64_t)row * a.hk + kh;
-  const bool writer = chunk == 0 && row < a.rows;
-  // walk this thread's tiles with the running counts: entry index and record slots
-  int run_pre[5];  // counts before the current tile, within the sequence
+  // the chunk's kept records
+  const int jend = min(tiles, (chunk + 1) * a.chunk);
+  for (int j = chunk * a.chunk; j < jend; ++j) {
+    if (j > 0 && j < runs.keep) continue;
+    const uint8_t *ks, *vs;
+    uint8_t *kd, *vd;
+    int kbytes, vbytes;
+    if (ex) {
+      const int64_t src = ((int64_t)s * a.nx + xs) * tiles + j;
+      const int64_t dst = a.ox + ((int64_t)s * a.nx + xs) * a.xstride + j;
+      ks = a.kx + src * KX_BYTES;
+      vs = a.vx + src * KX_BYTES;
+      kd = a.kxc + dst * KX_BYTES;
+      vd = a.vxc + dst * KX_BYTES;
+      kbytes = vbytes = dst < a.capx ? KX_BYTES : 0;
+    } else {
+      const int64_t src = hb_src * tiles + j, kn = kslot(j), vn = vslot(j);
+      const bool k4 = is4(j), v4 = !v8(j);
+      ks = k4 ? a.k4p + src * K4_BYTES : a.kp + src * K8_BYTES;
+      kd = k4 ? a.k4c + kn * K4_BYTES : a.k8c + kn * K8_BYTES;
+      kbytes = k4 ? (kn < a.cap4 && a.k4p != nullptr ? K4_BYTES : 0) : (kn < a.cap8 ? K8_BYTES : 0);
+      vs = v4 ? a.v4p + src * V4_BYTES : a.v8p + src * V8_BYTES;
+      vd = v4 ? a.v4c + vn * V4_BYTES : a.v8c + vn * V8_BYTES;
+      vbytes = v4 ? (vn < a.capv4 && a.v4p != nullptr ? V4_BYTES : 0) : (vn < a.capv8 ? V8_BYTES : 0);
+    }
+    constexpr int STEP = STORE_THREADS * 16, STEPS = KX_BYTES / STEP;
+    v4i kw[STEPS], vw[STEPS];
 #pragma unroll
-  for (int f = 0; f < 5; ++f) run_pre[f] = before_head[f] + field(my_prefix, f);
-  int e = field(my_prefix, 0);  // entry index of this thread's first kept tile in head kh
-  for (int j = j0; j < j1; ++j) {
-    const TileClass c = classify(sb + 2 * kh * g, g, ex, tiles, j);
-    if (c.kept) {
-      const int64_t k4slot = a.o4 + (int64_t)s * seq_total[1] + run_pre[1];
-      const int64_t k8slot = a.o8 + (int64_t)s * seq_total[2] + run_pre[2];
-      const int64_t v8slot = a.ov8 + (int64_t)s * seq_total[3] + run_pre[3];
-      const int64_t v4slot = a.ov4 + (int64_t)s * seq_total[4] + run_pre[4];
-      const int64_t kslot = c.is4 ? k4slot : c.is8 ? k8slot : 0;
-      const int64_t vslot = c.v8 ? v8slot : c.v4 ? v4slot : 0;
-      if (writer && e < a.maxn) {
-        const bool vi8 = j == 0 || tiles - 1 - j < NEAR_V8;
-        a.entry[hb * a.maxn + e] = j | (1 << 30) | (vi8 ? 1 << 29 : 0);
-        a.kinfo[hb * a.maxn + e] = (c.mask & 0xff) | (c.is4 ? 1 << 8 : 0) | (int)((uint32_t)kslot << 9);
-        a.slot[hb * a.maxn + e] = (int)vslot;
-      }
-      if (j / STORE_CHUNK == chunk) {
-        CopyDesc dsc;
-        if (ex) {
-          const int64_t src = ((int64_t)s * a.nx + xs) * tiles + j;
-          const int64_t dst = a.ox + ((int64_t)s * a.nx + xs) * a.xstride + j;
-          dsc.kind = 1;
-          dsc.ksrc = dsc.vsrc = src;
-          dsc.kdst = dsc.vdst = dst;
-          dsc.kbytes = dsc.vbytes = dst < a.capx ? KX_BYTES : 0;
-        } else {
-          dsc.kind = 0;
-          dsc.ksrc = hb_src * tiles + j;
-          dsc.kdst = kslot;
-          dsc.kbytes = c.is4 ? (k4slot < a.cap4 ? K4_BYTES : 0) : (k8slot < a.cap8 ? K8_BYTES : 0);
-          dsc.vsrc = hb_src * tiles + j;
-          dsc.vdst = vslot;
-          dsc.vbytes = c.v8 ? (v8slot < a.capv8 ? V8_BYTES : 0) : (v4slot < a.capv4 ? V4_BYTES : 0);
-          if (c.is4 && a.k4p == nullptr) dsc.kbytes = 0;
-          if (c.v4 && a.v4p == nullptr) dsc.vbytes = 0;
-        }
-        desc[j % STORE_CHUNK] = dsc;
-      }
-      ++e;
+    for (int i = 0; i < STEPS; ++i) {
+      const int off = i * STEP + tid * 16;
+      if (off < kbytes) kw[i] = *reinterpret_cast<const v4i*>(ks + off);
+      if (off < vbytes) vw[i] = *reinterpret_cast<const v4i*>(vs + off);
     }
-    run_pre[0] += c.kept;
-    run_pre[1] += c.is4;
-    run_pre[2] += c.is8;
-    run_pre[3] += c.v8;
-    run_pre[4] += c.v4;
-  }
-  if (writer) {
-    const int cnt = field(head_total, 0);
-    for (int i = cnt + tid; i < a.maxn; i += STORE_THREADS) {
-      a.entry[hb * a.maxn + i] = 0;
-      a.kinfo[hb * a.maxn + i] = 0;
-      a.slot[hb * a.maxn + i] = 0;
-    }
-    if (tid == 0) {
-      a.count[hb] = cnt;
-      if (a.xslot) a.xslot[hb] = ex ? (int)(a.ox + ((int64_t)s * a.nx + xs) * a.xstride) : -1;
-    }
-    for (int i = tid; i < a.tiles_max * 4; i += STORE_THREADS) {
-      a.ka_c[hb * a.tiles_max * 4 + i] = i < tiles * 4 ? a.ka[hb_src * tiles * 4 + i] : 1.f;
-      if (a.ka4_c) a.ka4_c[hb * a.tiles_max * 4 + i] = (i < tiles * 4 && a.ka4) ? a.ka4[hb_src * tiles * 4 + i] : 1.f;
-    }
-    for (int i = tid; i < 3 * D; i += STORE_THREADS) {
-      a.kstat_c[hb * 3 * D + i] = a.kstat[hb_src * 3 * D + i];
-      a.vstat_c[hb * 3 * D + i] = a.vstat[hb_src * 3 * D + i];
-    }
-    if (kh == 0) {
-      if (tid == 0) a.prompt[row] = a.t;
-      for (int j = tid; j < a.tiles_max; j += STORE_THREADS)
-        a.fmt[(int64_t)row * a.tiles_max + j] = (j < tiles && !(j == 0 || tiles - 1 - j < NEAR_V8)) ? 2 : 1;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const int off = i * STEP + tid * 16;
+      if (off < kbytes) *reinterpret_cast<v4i*>(kd + off) = kw[i];
+      if (off < vbytes) *reinterpret_cast<v4i*>(vd + off) = vw[i];
     }
   }
-  __syncthreads();
-  // copy the chunk's kept records, one tile after another, 16 bytes per thread per step
-  const int nt = min(STORE_CHUNK, tiles - chunk * STORE_CHUNK);
-  for (int i = 0; i < nt; ++i) {
-    const CopyDesc d = desc[i];
-    const uint8_t* ks = d.kind ? a.kx + d.ksrc * KX_BYTES
-                               : (d.kbytes == K4_BYTES ? a.k4p + d.ksrc * K4_BYTES : a.kp + d.ksrc * K8_BYTES);
-    uint8_t* kd = d.kind ? a.kxc + d.kdst * KX_BYTES
-                         : (d.kbytes == K4_BYTES ? a.k4c + d.kdst * K4_BYTES : a.k8c + d.kdst * K8_BYTES);
-    for (int off = tid * 16; off < d.kbytes; off += STORE_THREADS * 16)
-      *reinterpret_cast<uint4*>(kd + off) = *reinterpret_cast<const uint4*>(ks + off);
-    const uint8_t* vs = d.kind ? a.vx + d.vsrc * KX_BYTES
-                               : (d.vbytes == V4_BYTES ? a.v4p + d.vsrc * V4_BYTES : a.v8p + d.vsrc * V8_BYTES);
-    uint8_t* vd = d.kind ? a.vxc + d.vdst * KX_BYTES
-                         : (d.vbytes == V4_BYTES ? a.v4c + d.vdst * V4_BYTES : a.v8c + d.vdst * V8_BYTES);
-    for (int off = tid * 16; off < d.vbytes; off += STORE_THREADS * 16)
-      *reinterpret_cast<uint4*>(vd + off) = *reinterpret_cast<const uint4*>(vs + off);
+  if (chunk != 0 || row >= a.rows) return;
+  // the head's metadata row
+  const int cnt = 1 + tiles - runs.keep;
+  for (int e = tid; e < a.maxn; e += STORE_THREADS) {
+    int entry = 0, info = 0, slot = 0;
+    if (e < cnt) {
+      const int j = e == 0 ? 0 : runs.keep + e - 1, d = tiles - 1 - j;
+      int mask = 0;
+      for (int r = 0; r < g; ++r) {
+        const bool on = ex || j == 0 || d < sb[2 * (kh * g + r)] || d < sb[2 * (kh * g + r) + 1];
+        mask |= (on ? 1 : 0) << r;
+      }
+      entry = j | (1 << 30) | (j == 0 || d < NEAR_V8 ? 1 << 29 : 0);
+      info = (mask & 0xff) | (is4(j) ? 1 << 8 : 0) | (int)((uint32_t)(ex ? 0 : kslot(j)) << 9);
+      slot = ex ? 0 : (int)vslot(j);
+    }
+    a.entry[hb * a.maxn + e] = entry;
+    a.kinfo[hb * a.maxn + e] = info;
+    a.slot[hb * a.maxn + e] = slot;
+  }
+  if (tid == 0) {
+    a.count[hb] = cnt;
+    if (a.xslot) a.xslot[hb] = ex ? (int)(a.ox + ((int64_t)s * a.nx + xs) * a.xstride) : -1;
+  }
+  for (int i = tid; i < a.tiles_max * 4; i += STORE_THREADS) {
+    a.ka_c[hb * a.tiles_max * 4 + i] = i < tiles * 4 ? a.ka[hb_src * tiles * 4 + i] : 1.f;
+    if (a.ka4_c) a.ka4_c[hb * a.tiles_max * 4 + i] = (i < tiles * 4 && a.ka4) ? a.ka4[hb_src * tiles * 4 + i] : 1.f;
+  }
+  for (int i = tid; i < 3 * D; i += STORE_THREADS) {
+    a.kstat_c[hb * 3 * D + i] = a.kstat[hb_src * 3 * D + i];
+    a.vstat_c[hb * 3 * D + i] = a.vstat[hb_src * 3 * D + i];
+  }
+  if (kh == 0) {
+    if (tid == 0) a.prompt[row] = a.t;
+    for (int j = tid; j < a.tiles_max; j += STORE_THREADS)
+      a.fmt[(int64_t)row * a.tiles_max + j] = (j < tiles && !(j == 0 || tiles - 1 - j < NEAR_V8)) ? 2 : 1;
   }
 }
 
