@@ -567,7 +567,9 @@ class DecodeCache:
         key = ("plan", _geometry(q), _geometry(k), _geometry(out), float(scale))
         if key not in e:
             hq = q.shape[1]
-            if self.tasks and e["xslot"] is None and "tasks" not in e and hasattr(self.module, "decode_tasks"):
+            # (a growing cache with exact heads gathers: tail_spill keeps no task rows for exact heads)
+            if self.tasks and "tasks" not in e and hasattr(self.module, "decode_tasks") and \
+                    (e["xslot"] is None or not e["grow_splits"]):
                 layout = e["layout"]
                 if "items" not in layout:
                     items_host = self._task_items(e)
