@@ -215,9 +215,13 @@ class Prefill:
         kx = vx = None
         if exact is not None:
             kx, vx = self.exact_records(batch * nx * rows * KX_BYTES, device)
-        self.module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"],
-                            ops["q4"], ops["qa4"], ops["k4"], ops["ka4"], k4x, ops["vpartial"], ops["vstat"],
-                            packed[F16], packed[I8], packed[I4], v8sum, exact, nx, kx, vx)
+        if nx == hk and decode is None:
+            # (every KV head exact and no cache to fill: nothing reads the quantized operands)
+            self.module.pack_exact(k, v, exact, nx, kx, vx)
+        else:
+            self.module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"],
+                                ops["q4"], ops["qa4"], ops["k4"], ops["ka4"], k4x, ops["vpartial"], ops["vstat"],
+                                packed[F16], packed[I8], packed[I4], v8sum, exact, nx, kx, vx)
         out = None
         if attend:
             dtype = self.out_dtype or q.dtype
