@@ -72,16 +72,100 @@ __device__ __forceinline__ v4i k_frag(const uint8_t* __restrict__ k_lds, int F, 
   }
 }
 
+// An fp16 tile (KF16; prefill_sm80.cu:358-383) in two parts, so that its V record may still be on its way
+// while the first runs: INT8 scores, masked where `masked`, the running maximum and the fp16 probabilities
+// p; then P V.
+__device__ __forceinline__ void f16_probs(const PrefillArgs& a, PrefillState& st, const v4i (&qf)[4], float qs,
+                                          const float (&ks)[4], int col, bool masked, int qrow,
+                                          const uint8_t* __restrict__ k_lds, v8h (&p)[2][2]) {
+  const int L = threadIdx.x & 63, half = L >> 5;
+  // ---- S^T = K Q^T over 128 features, two 32-key blocks
+  v16i s[2];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[kb][r] = (int)MAGIC_BITS;
+#pragma unroll
+  for (int kstep = 0; kstep < 4; ++kstep)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) s[kb] = mfma_i8(k_frag<KF16>(k_lds, kb * 4 + kstep, L), qf[kstep], s[kb]);
+  // score of accumulator r of block kb: the magic float 1.5*2^23 + dot
+  auto score = [&](int kb, int r) -> float {
+    float v = __int_as_float(s[kb][r]);
+    if (masked) {
+      const int key = col * BN + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (key > qrow || key >= a.t) v = -__builtin_inff();
+    }
+    return v;
+  };
+  // ---- scaled row max (prefill_sm80.cu:244-253)
+  float slope[4];
+#pragma unroll
+  for (int gi = 0; gi < 4; ++gi) slope[gi] = qs * ks[gi];
+  float tile = -__builtin_inff();
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int hg = 0; hg < 2; ++hg) {
+      float mx = score(kb, hg * 8);
+#pragma unroll
+      for (int r = 1; r < 8; ++r) mx = fmaxf(mx, score(kb, hg * 8 + r));
+      if (mx > -__builtin_inff()) tile = fmaxf(tile, slope[kb * 2 + hg] * (mx - MAGIC));
+    }
+  tile = xor32_max(tile);
+  // (fp16 tiles need the exact running max: their P is relative to it)
+  const float n = fmaxf(st.m, tile);
+  const float alpha = texp2(st.m - n);
+  st.m = n;
+  if (__any(alpha != 1.f)) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st.acc[cb][r] *= alpha;
+  }
+  st.den *= alpha;
+  float c[4];
+#pragma unroll
+  for (int gi = 0; gi < 4; ++gi) c[gi] = __builtin_fmaf(-slope[gi], MAGIC, -st.m);
+  float psum = 0.f;
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int gi = kb * 2 + (r >> 3);
+      // (a zero query row has slope 0, and 0 * -inf of a masked key is NaN: the clamp turns it
+      // into 2^-125, which rounds to fp16 0 as the masked key's probability must)
+      const _Float16 h = (_Float16)pexp2(fmaxf(__builtin_fmaf(slope[gi], score(kb, r), c[gi]), -125.f));
+      p[kb][r >> 3][r & 7] = h;
+      psum += (float)h;
+    }
+  st.den += xor32_add(psum);
+}
+__device__ __forceinline__ void f16_pv(PrefillState& st, const v8h (&p)[2][2], const uint8_t* __restrict__ v_lds,
+                                       const uint8_t* __restrict__ v_hi) {
+  const int L = threadIdx.x & 63;
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int kh = 0; kh < 2; ++kh) {
+        // fp16 V record: fragments 0..7 in v_lds, 8..15 in v_hi
+        const int F = (cb * 2 + kb) * 2 + kh;
+        const v8h vf = *reinterpret_cast<const v8h*>((F < 8 ? v_lds : v_hi) + (F & 7) * 1024 + L * 16);
+        st.acc[cb] = mfma_f16(vf, p[kb][kh], st.acc[cb]);
+      }
+}
+
 // SUMS: the quantized P V accumulators start from the tile's -127 * sum(V8) in LDS (vs_lds, channel
 // order) instead of two MFMAs against a constant -127 operand.  QMASK: a quantized tile that is the
 // query tile itself (an INT4 list that reaches the diagonal, w8 = 0): keys past the query row or
 // past t get level 0 and stay out of the tile max, as fp16 tiles mask them.
-template <int KIND, bool SUMS = false, bool QMASK = false>
+template <int KIND, bool SUMS, bool QMASK>
 __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillState& st, const v4i (&qf)[4], float qs,
-                                             const float (&ks)[4], int col, bool masked, int qrow,
+                                             const float (&ks)[4], int col, int qrow,
                                              const uint8_t* __restrict__ k_lds, const uint8_t* __restrict__ v_lds,
-                                             const uint8_t* __restrict__ v_hi = nullptr,
-                                             const int32_t* __restrict__ vs_lds = nullptr) {
+                                             const int32_t* __restrict__ vs_lds) {
   constexpr bool IS4 = KIND == KQ4 || KIND == KQ4X;  // INT4 arithmetic (16 * dot)
   const int L = threadIdx.x & 63, half = L >> 5;
   // ---- S^T = K Q^T over 128 features, two 32-key blocks
@@ -110,17 +194,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillState&
 
   // score of accumulator r of block kb as a float: the magic float for 8-bit
   // codes (1.5*2^23 + dot), 16*dot for 4-bit codes (the MFMA saw 16*code keys;
-  // the 1/16 is folded into the slope, which is exact).  fp16 tiles mask here.
-  auto score = [&](int kb, int r) -> float {
-    float v = IS4 ? (float)s[kb][r] : __int_as_float(s[kb][r]);
-    if constexpr (KIND == KF16) {
-      if (masked) {
-        const int key = col * BN + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (key > qrow || key >= a.t) v = -__builtin_inff();
-      }
-    }
-    return v;
-  };
+  // the 1/16 is folded into the slope, which is exact).
+  auto score = [&](int kb, int r) -> float { return IS4 ? (float)s[kb][r] : __int_as_float(s[kb][r]); };
 
   // ---- scaled row max (prefill_sm80.cu:244-253)
   float slope[4];
@@ -131,37 +206,29 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillState&
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int hg = 0; hg < 2; ++hg) {
-      if constexpr (KIND == KF16) {
-        float mx = score(kb, hg * 8);
-#pragma unroll
-        for (int r = 1; r < 8; ++r) mx = fmaxf(mx, score(kb, hg * 8 + r));
-        if (mx > -__builtin_inff()) tile = fmaxf(tile, slope[kb * 2 + hg] * (mx - MAGIC));
-      } else {
-        // the group's largest integer accumulator (the magic-offset dot product, or 16 * dot), whose
-        // order is the scores' order, converted once (under QMASK a group with no valid key, all
-        // INT_MIN, leaves the tile max alone)
-        const int g0 = hg * 8;
-        int mx = max(max(s[kb][g0], s[kb][g0 + 1]), s[kb][g0 + 2]);
-        mx = max(max(mx, s[kb][g0 + 3]), s[kb][g0 + 4]);
-        mx = max(max(mx, s[kb][g0 + 5]), s[kb][g0 + 6]);
-        mx = max(mx, s[kb][g0 + 7]);
-        // (|dot| < 2^22: the magic float minus 1.5 * 2^23 is the dot product exactly)
-        const float d = IS4 ? (float)mx : __int_as_float(mx) - MAGIC;
-        if (!QMASK || mx != INT_MIN) tile = fmaxf(tile, slope[kb * 2 + hg] * d);
-      }
+      // the group's largest integer accumulator (the magic-offset dot product, or 16 * dot), whose
+      // order is the scores' order, converted once (under QMASK a group with no valid key, all
+      // INT_MIN, leaves the tile max alone)
+      const int g0 = hg * 8;
+      int mx = max(max(s[kb][g0], s[kb][g0 + 1]), s[kb][g0 + 2]);
+      mx = max(max(mx, s[kb][g0 + 3]), s[kb][g0 + 4]);
+      mx = max(max(mx, s[kb][g0 + 5]), s[kb][g0 + 6]);
+      mx = max(mx, s[kb][g0 + 7]);
+      // (|dot| < 2^22: the magic float minus 1.5 * 2^23 is the dot product exactly)
+      const float d = IS4 ? (float)mx : __int_as_float(mx) - MAGIC;
+      if (!QMASK || mx != INT_MIN) tile = fmaxf(tile, slope[kb * 2 + hg] * d);
     }
   tile = xor32_max(tile);
-  // Running reference max.  fp16 tiles need the exact running max (their P
-  // is relative to it).  INT8/INT4 P levels are relative to the tile's own
+  // Running reference max.  INT8/INT4 P levels are relative to the tile's own
   // base, so the reference max only scales acc and den alike and acc/den does
-  // not depend on it: those tiles move it only when a tile exceeds it by more
-  // than 64, which skips most rescales.  Headroom: bq <= 2^(64 + margin)/255
+  // not depend on it: it moves only when a tile exceeds it by more than 64,
+  // which skips most rescales.  Headroom: bq <= 2^(64 + margin)/255
   // and |PV| < 2^21 per tile, so acc stays below 2^(64 + 21 + 11) over 2048
   // tiles, far inside fp32.
-  const float n = KIND == KF16 ? fmaxf(st.m, tile) : (tile > st.m + 64.f ? tile : st.m);
-  // (quantized tiles rarely move the max: the factor and the rescale only when some row's does)
+  const float n = tile > st.m + 64.f ? tile : st.m;
+  // (tiles rarely move the max: the factor and the rescale only when some row's does)
   float alpha = 1.f;
-  if (KIND == KF16 || __any(n != st.m)) alpha = texp2(st.m - n);
+  if (__any(n != st.m)) alpha = texp2(st.m - n);
   st.m = n;
   if (__any(alpha != 1.f)) {
 #pragma unroll
@@ -170,94 +237,61 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillState&
       for (int r = 0; r < 16; ++r) st.acc[cb][r] *= alpha;
   }
 
-  if constexpr (KIND == KF16) {
-    // ---- fp16 P x fp16 V' (prefill_sm80.cu:358-383)
-    st.den *= alpha;
-    float c[4];
+  // ---- quantized P (u8) x INT8 V' (prefill_sm80.cu:384-449)
+  const float ksmax = max_arith(max3_arith(ks[0], ks[1], ks[2]), ks[3]);
+  float base = tile > -__builtin_inff() ? tile : st.m;
+  base += __builtin_fmaf(qs * ksmax, 0.75f, fabsf(base) * 2.4e-7f);
+  // the reference divides by the level count under fast math; here: times its rounded reciprocal
+  const float bq = texp2(base - st.m) * (1.f / 255.f);
+  float c[4];
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) c[gi] = __builtin_fmaf(-slope[gi], MAGIC, -st.m);
-    v8h p[2][2];
-    float psum = 0.f;
+  for (int gi = 0; gi < 4; ++gi)
+    c[gi] = KIND == KI8 ? __builtin_fmaf(-slope[gi], MAGIC, -base) : -base;
+  uint32_t pw[2][4];
+  int rsn = 0;  // sum of this lane's 32 bytes 127 - P (signed dot product of the s8 operand words)
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+  for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int gi = kb * 2 + (r >> 3);
-        // (a zero query row has slope 0, and 0 * -inf of a masked key is NaN: the clamp turns it
-        // into 2^-125, which rounds to fp16 0 as the masked key's probability must)
-        const _Float16 h = (_Float16)pexp2(fmaxf(__builtin_fmaf(slope[gi], score(kb, r), c[gi]), -125.f));
-        p[kb][r >> 3][r & 7] = h;
-        psum += (float)h;
+    for (int qd = 0; qd < 4; ++qd) {
+      uint32_t y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = qd * 4 + i, gi = kb * 2 + (r >> 3);
+        float e = pexp2(__builtin_fmaf(slope[gi], score(kb, r), c[gi]));
+        if constexpr (QMASK) e = s[kb][r] == INT_MIN ? 0.f : e;
+        y[i] = __float_as_uint(__builtin_fmaf(e, 255.f, PMAGIC_HALF));
       }
-    st.den += xor32_add(psum);
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-          // fp16 V record: fragments 0..7 in v_lds, 8..15 in v_hi
-          const int F = (cb * 2 + kb) * 2 + kh;
-          const v8h vf = *reinterpret_cast<const v8h*>((F < 8 ? v_lds : v_hi) + (F & 7) * 1024 + L * 16);
-          st.acc[cb] = mfma_f16(vf, p[kb][kh], st.acc[cb]);
-        }
-  } else {
-    // ---- quantized P (u8) x INT8 V' (prefill_sm80.cu:384-449)
-    const float ksmax = max_arith(max3_arith(ks[0], ks[1], ks[2]), ks[3]);
-    float base = tile > -__builtin_inff() ? tile : st.m;
-    base += __builtin_fmaf(qs * ksmax, 0.75f, fabsf(base) * 2.4e-7f);
-    // the reference divides by the level count under fast math; here: times its rounded reciprocal
-    const float bq = texp2(base - st.m) * (1.f / 255.f);
-    float c[4];
-#pragma unroll
-    for (int gi = 0; gi < 4; ++gi)
-      c[gi] = KIND == KI8 ? __builtin_fmaf(-slope[gi], MAGIC, -base) : -base;
-    uint32_t pw[2][4];
-    int rsn = 0;  // sum of this lane's 32 bytes 127 - P (signed dot product of the s8 operand words)
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        uint32_t y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = qd * 4 + i, gi = kb * 2 + (r >> 3);
-          float e = pexp2(__builtin_fmaf(slope[gi], score(kb, r), c[gi]));
-          if constexpr (QMASK) e = s[kb][r] == INT_MIN ? 0.f : e;
-          y[i] = __float_as_uint(__builtin_fmaf(e, 255.f, PMAGIC_HALF));
-        }
-        pw[kb][qd] = pack_byte1(y[0], y[1], y[2], y[3]) ^ 0x7f7f7f7fu;  // 127 - P as s8
-        rsn = __builtin_amdgcn_sdot4((int)pw[kb][qd], 0x01010101, rsn, false);
-      }
-    // the row's 64 levels: 2 * 32 * 127 minus the sum of 127 - P over lanes L and L ^ 32 (mod 2^32)
-    const uint32_t rs = 8128u - xor32_add((uint32_t)rsn);
-    st.den = __builtin_fmaf((float)rs, bq, st.den * alpha);
-    const v4i neg127 = {(int)0x81818181u, (int)0x81818181u, (int)0x81818181u, (int)0x81818181u};
-    const v4i b0 = {(int)pw[0][0], (int)pw[0][1], (int)pw[0][2], (int)pw[0][3]};
-    const v4i b1 = {(int)pw[1][0], (int)pw[1][1], (int)pw[1][2], (int)pw[1][3]};
-    const float nbq = -bq;
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      const v4i va = *reinterpret_cast<const v4i*>(v_lds + (cb * 2 + 0) * 1024 + L * 16);
-      const v4i vb = *reinterpret_cast<const v4i*>(v_lds + (cb * 2 + 1) * 1024 + L * 16);
-      v16i d = {};
-      if constexpr (SUMS) {
-        // accumulator r of channel block cb is channel cb*32 + 8*(r/4) + 4*half + r%4
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const v4i w = *reinterpret_cast<const v4i*>(vs_lds + cb * 32 + 8 * j + 4 * half);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) d[4 * j + i] = w[i];
-        }
-      } else {
-        d = mfma_i8(va, neg127, d);
-        d = mfma_i8(vb, neg127, d);
-      }
-      d = mfma_i8(va, b0, d);
-      d = mfma_i8(vb, b1, d);  // = -sum_k P_k v_k
-#pragma unroll
-      for (int r = 0; r < 16; ++r) st.acc[cb][r] = __builtin_fmaf((float)d[r], nbq, st.acc[cb][r]);
+      pw[kb][qd] = pack_byte1(y[0], y[1], y[2], y[3]) ^ 0x7f7f7f7fu;  // 127 - P as s8
+      rsn = __builtin_amdgcn_sdot4((int)pw[kb][qd], 0x01010101, rsn, false);
     }
+  // the row's 64 levels: 2 * 32 * 127 minus the sum of 127 - P over lanes L and L ^ 32 (mod 2^32)
+  const uint32_t rs = 8128u - xor32_add((uint32_t)rsn);
+  st.den = __builtin_fmaf((float)rs, bq, st.den * alpha);
+  const v4i neg127 = {(int)0x81818181u, (int)0x81818181u, (int)0x81818181u, (int)0x81818181u};
+  const v4i b0 = {(int)pw[0][0], (int)pw[0][1], (int)pw[0][2], (int)pw[0][3]};
+  const v4i b1 = {(int)pw[1][0], (int)pw[1][1], (int)pw[1][2], (int)pw[1][3]};
+  const float nbq = -bq;
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const v4i va = *reinterpret_cast<const v4i*>(v_lds + (cb * 2 + 0) * 1024 + L * 16);
+    const v4i vb = *reinterpret_cast<const v4i*>(v_lds + (cb * 2 + 1) * 1024 + L * 16);
+    v16i d = {};
+    if constexpr (SUMS) {
+      // accumulator r of channel block cb is channel cb*32 + 8*(r/4) + 4*half + r%4
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const v4i w = *reinterpret_cast<const v4i*>(vs_lds + cb * 32 + 8 * j + 4 * half);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[4 * j + i] = w[i];
+      }
+    } else {
+      d = mfma_i8(va, neg127, d);
+      d = mfma_i8(vb, neg127, d);
+    }
+    d = mfma_i8(va, b0, d);
+    d = mfma_i8(vb, b1, d);  // = -sum_k P_k v_k
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st.acc[cb][r] = __builtin_fmaf((float)d[r], nbq, st.acc[cb][r]);
   }
 }
 
@@ -540,7 +574,11 @@ __global__ __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(2))
   const float* ka8 = a.ka + rec0 * 4;
   const float* ka4p = a.ka4 ? a.ka4 + rec0 * 4 : nullptr;
 
-  // ---- F16 pass: tile 0, then the diagonal tile when qb > 0 (synchronous staging; pair 0)
+  // ---- F16 pass: tile 0, then the diagonal tile when qb > 0 (pair 0).  Both K records and tile 0's V come
+  // together; the diagonal's V (which takes both V buffers, as tile 0's does) follows once every wave is done
+  // with tile 0 and arrives while its scores and probabilities are computed.  (Against copying each tile's K and V
+  // before it: four uniform-band prompts of 4,096 tokens 500 -> 492 us, 1,024 tokens 39.5 -> 39.0 us, 30,001 banded
+  // tokens 1776 -> 1762 us.)
   const int nf16 = qb > 0 ? 2 : 1;
   // this pair's part [q0, q1) of the quantized tile list (INT8 tiles, then INT4 ones): with two pairs,
   // pair 0's F16 tiles (each priced as two quantized ones: their copies are synchronous) and quantized
@@ -549,21 +587,36 @@ __global__ __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(2))
   const int total = n8 + n4;
   const int c = PAIRS == 2 ? max(0, (total - 2 * nf16 + 1) / 2) : total;
   const int q0 = pair == 0 ? 0 : c, q1 = pair == 0 ? c : total;
-  // barriers each pair passes: two per F16 tile, one before its quantized part and one per tile of it
-  const int bar0 = 2 * nf16 + (c > 0 ? 1 + c : 0), bar1 = total > c ? 1 + total - c : 0;
-  for (int i = 0; i < (pair == 0 ? nf16 : 0); ++i) {
-    const int col = i == 0 ? 0 : qb;
-    __syncthreads();
-    // (with the first copy: the epilogue's V mean and scale, 1 KiB, so that it reads them from LDS)
-    if (i == 0 && tid < 64)
+  // barriers each pair passes: one for tile 0, two more for the diagonal, one before its quantized part and one
+  // per tile of it
+  const int bar0 = 2 * nf16 - 1 + (c > 0 ? 1 + c : 0), bar1 = total > c ? 1 + total - c : 0;
+  if (pair == 0) {
+    // (with the first copies: the epilogue's V mean and scale, 1 KiB, so that it reads them from LDS)
+    if (tid < 64)
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(a.vstat + ((int64_t)b * a.hk + kh) * 3 * D + tid * 4),
                                        (__attribute__((address_space(3))) void*)(vms_lds + tid * 4), 16, 0, 0);
-    lds_copy_async<K8_BYTES>(a.k8 + (rec0 + col) * K8_BYTES, k_lds0[0]);
-    lds_copy_async<V16_BYTES / 2>(a.v16 + (rec0 + col) * V16_BYTES, v_lds0[0]);
-    lds_copy_async<V16_BYTES / 2>(a.v16 + (rec0 + col) * V16_BYTES + V16_BYTES / 2, v_lds1[0]);
+    auto copy_v16 = [&](int col) __attribute__((always_inline)) {
+      lds_copy_async<V16_BYTES / 2>(a.v16 + (rec0 + col) * V16_BYTES, v_lds0[0]);
+      lds_copy_async<V16_BYTES / 2>(a.v16 + (rec0 + col) * V16_BYTES + V16_BYTES / 2, v_lds1[0]);
+    };
+    lds_copy_async<K8_BYTES>(a.k8 + rec0 * K8_BYTES, k_lds0[0]);
+    copy_v16(0);
+    if (nf16 == 2) lds_copy_async<K8_BYTES>(a.k8 + (rec0 + qb) * K8_BYTES, k_lds1[0]);
+    v8h p[2][2];
     lds_wait();
-    const float ks[4] = {ka8[col * 4], ka8[col * 4 + 1], ka8[col * 4 + 2], ka8[col * 4 + 3]};
-    prefill_tile<KF16>(a, st, qf, qs8, ks, col, i == nf16 - 1 && col == qb, qrow, k_lds0[0], v_lds0[0], v_lds1[0]);
+    {
+      const float ks[4] = {ka8[0], ka8[1], ka8[2], ka8[3]};
+      f16_probs(a, st, qf, qs8, ks, 0, nf16 == 1, qrow, k_lds0[0], p);
+      f16_pv(st, p, v_lds0[0], v_lds1[0]);
+    }
+    if (nf16 == 2) {
+      __syncthreads();  // every wave is done with tile 0's V
+      copy_v16(qb);
+      const float ks[4] = {ka8[qb * 4], ka8[qb * 4 + 1], ka8[qb * 4 + 2], ka8[qb * 4 + 3]};
+      f16_probs(a, st, qf, qs8, ks, qb, true, qrow, k_lds1[0], p);
+      lds_wait();
+      f16_pv(st, p, v_lds0[0], v_lds1[0]);
+    }
   }
 
   // ---- INT8 then INT4 passes as one pipelined tile list: the next tile's
@@ -668,8 +721,8 @@ __global__ __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(2))
       const float4 k4v = *reinterpret_cast<const float4*>(vkc + VK + (KIND == KI8 ? 0 : 4));
       const float ks[4] = {k4v.x, k4v.y, k4v.z, k4v.w};
       constexpr bool QMASK = decltype(mask)::value != 0;
-      if constexpr (KIND == KI8) prefill_tile<KI8, SUMS>(a, st, qf, qs8, ks, col, false, qrow, kc, vc, nullptr, vkc);
-      else prefill_tile<KIND, SUMS, QMASK>(a, st, q4f, qs4, ks, col, QMASK, qrow, kc, vc, nullptr, vkc);
+      if constexpr (KIND == KI8) prefill_tile<KI8, SUMS, false>(a, st, qf, qs8, ks, col, qrow, kc, vc, vkc);
+      else prefill_tile<KIND, SUMS, QMASK>(a, st, q4f, qs4, ks, col, qrow, kc, vc, vkc);
     };
     // Tiles [i, end) of one kind, the first in buffer set PARITY.  Each kind has a
     // loop of its own: with both kinds in one loop body the compiler copies the
