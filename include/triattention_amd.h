@@ -323,8 +323,8 @@ int tri_decode_occupancy(int* blocks);
 int tri_device_cus(int* cus);
 
 /* Extension, no counterpart in the reference: the launch form of tri_attention for this process.
- * mode 0 (default): launches with at most two workgroups per compute unit take four-wave workgroups
- * whose two wave pairs split each query tile's key tiles (the F16 tiles and the start of the
+ * mode 0 (default): launches with at most two workgroups per compute unit (four, when batch * hq is at
+ * most an eighth of the compute units and no head is exact) take four-wave workgroups whose two wave pairs split each query tile's key tiles (the F16 tiles and the start of the
  * quantized list, and the rest), merged before the output; larger launches take two-wave
  * workgroups.  mode 1: always two-wave workgroups; mode 2: always four.  Both forms follow the
  * reference's per-tile arithmetic; they differ only in the fp32 summation order across the two

@@ -327,13 +327,20 @@ int tri_attention(const int32_t* order, int n_order, const int32_t* bands, int b
   a.k4x = static_cast<const uint8_t*>(k4x);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Launches of at most two workgroups per CU (short prompts) leave SIMDs without a wave: each
-  // workgroup then takes four waves, two pairs that split its key tiles (prefill_kernel<., 2>).
+  // workgroup then takes four waves, two pairs that split its key tiles (prefill_kernel<., 2>).  Up to four per
+  // CU the longest rows' serial tile lists still set the time when few (sequence, q-head) rows hold them
+  // (batch * hq <= CUs / 8), and splitting them pays (whole Prefill calls, two-wave / four-wave workgroups:
+  // 2,048 tokens Hq 28 79.0 / 75.2 us, Hq 24 76.9 / 71.0, Hq 32 82.5 / 80.6; 1,400 tokens Hq 24 59.0 / 49.4), not
+  // beyond (3,000 tokens Hq 28 109 / 112; 4,096 158 / 168), not for more, shorter rows (4 x 512 tokens Hq 24
+  // 50.5 / 58.2), and not with exact heads, whose tiles are not split (2,047 tokens, all exact, 79 / 86).
   const int pmode = g_prefill_pairs.load();
   bool pairs = pmode == 2;
   if (pmode == 0) {
     int cus = 0;
     if (device_cus(&cus) != 0) return 1;
-    pairs = (int64_t)n_order * batch <= 2 * (int64_t)cus;
+    const int64_t wgs = (int64_t)n_order * batch;
+    pairs = wgs <= 2 * (int64_t)cus ||
+            (exact == nullptr && wgs <= 4 * (int64_t)cus && (int64_t)batch * hq * 8 <= (int64_t)cus);
   }
   const dim3 grid(n_order, batch);
   if (pairs) {
