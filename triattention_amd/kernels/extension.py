@@ -139,10 +139,14 @@ class Module:
 
     # -------------------------------------------------------------- prepare_qk
     @staticmethod
-    def _check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x):
+    def _check_rows(q, k):
         _check(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 4 and q.size(3) == D and q.stride(3) == 1 and
                k.dtype == torch.bfloat16 and k.dim() == 4 and k.size(0) == q.size(0) and k.size(2) == q.size(2) and
                k.size(3) == D and k.stride(3) == 1, "BF16 Q/K [B,H,T,128] with contiguous features")
+
+    @staticmethod
+    def _check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x):
+        Module._check_rows(q, k)
         b, hq, t, _ = q.shape
         hk = k.size(1)
         tiles = (t + 63) // 64
@@ -268,8 +272,14 @@ class Module:
                      int(nx) if exact is not None else 0, _ptr(v8sum), _ptr(k4x))
         return out
 
-    def pack_exact(self, k, v, exact, nx, kx, vx):
-        """bf16 K/V of the exact KV heads -> KX/VX records [B][nx][tiles] (16 KiB each; extension)."""
+    def pack_exact(self, k, v, exact, nx, kx, vx, q=None):
+        """bf16 K/V of the exact KV heads -> KX/VX records [B][nx][tiles] (16 KiB each; extension).
+
+        ``q``: the queries that will attend to them where no ``prepare`` checks that they and K are of one
+        prompt, on one device."""
+        if q is not None:
+            self._check_rows(q, k)
+            _check(k.device == v.device == q.device, "Q/K/V on one device")
         b, h, hk, t = self._check_exact(k, v, exact, nx, kx, vx)
         self._launch(k.device, self.lib.tri_pack_exact, _ptr(k), *k.stride()[:3], _ptr(v), *v.stride()[:3], b, h, hk,
                      t, _ptr(exact), int(nx), _ptr(kx), _ptr(vx))

@@ -217,7 +217,7 @@ class Prefill:
             kx, vx = self.exact_records(batch * nx * rows * KX_BYTES, device)
         if nx == hk and decode is None:
             # (every KV head exact and no cache to fill: nothing reads the quantized operands)
-            self.module.pack_exact(k, v, exact, nx, kx, vx)
+            self.module.pack_exact(k, v, exact, nx, kx, vx, q=q)
         else:
             self.module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"],
                                 ops["q4"], ops["qa4"], ops["k4"], ops["ka4"], k4x, ops["vpartial"], ops["vstat"],
