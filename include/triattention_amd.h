@@ -136,7 +136,8 @@ int tri_pack_exact(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, cons
  * listed splits and reads each one's entries, record offsets and K scales from the table (one memory
  * round trip) instead of gathering them; the partials of splits the table leaves out are not written,
  * so the caller holds them at the empty partial (pm = -FLT_MAX, pl = 0, po = 0).  Ignored for a cache
- * with exact heads (xslot set).
+ * with exact heads (xslot set), unless n_tasks is minus the number of listed splits and tail_base is NULL:
+ * the table then lists the exact heads' splits too.
  * Tail growth (extension): tail_base NULL keeps the reference's tail (it holds step tokens before the
  * new one, and past max_tail - 1 the new token overwrites the last slot, common_device.cuh:384);
  * otherwise int64 on the device, the tokens tri_tail_spill has moved from the tail into the cache since

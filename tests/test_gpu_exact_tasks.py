@@ -35,3 +35,31 @@ def test_task_table_equals_the_gather(module, hq, hk, exact, prompts, per):
         outs.append(cache(0, q, k, v, 128 ** -0.5).clone())
         assert ("tasks" in cache.layers[0]) == tasks
     assert torch.equal(*outs)
+
+
+def test_a_table_is_ignored_with_exact_heads_unless_it_says_that_it_lists_them(module, monkeypatch):
+    """n_tasks > 0 with xslot gathers: a table of one split and partials never cleared change nothing."""
+    g = S.gen(9600)
+    cache = DecodeCache(module, max_tail=4)
+    cache.out_dtype = torch.float32
+    bands = torch.tensor([[S.INF, S.INF]] * 3 + [[1, S.INF]] * 3, dtype=torch.int32)
+    pk, pv = (S.outlier_tensor(g, 1, 2, 900).cuda() for _ in range(2))
+    Prefill(module, bands_fn_of(bands, [1]), cache).store_only(0, pk, pv, 6)
+    calls = []
+    real = module.plan_decode
+    monkeypatch.setattr(module, "plan_decode", lambda *a, **kw: calls.append((a, kw)) or real(*a, **kw))
+    q, k, v = (S.outlier_tensor(g, 1, h, 1).cuda() for h in (6, 2, 2))
+    cache(0, q, k, v, 128 ** -0.5)
+    args, kw = calls[-1]
+    args = list(args)
+    table, n = args[30]
+    assert kw["exact_tasks"] and n > 1
+    outs = []
+    for tasks, exact_tasks in (((table, n), True), ((table[:512], 1), False)):
+        if not exact_tasks:
+            args[20:23] = [torch.full_like(x, 7.0) for x in args[20:23]]
+        args[19] = torch.empty_like(args[19])
+        args[30], kw["exact_tasks"] = tasks, exact_tasks
+        real(*args, **kw).run(q, k, v, args[19])
+        outs.append(args[19])
+    assert torch.equal(*outs)

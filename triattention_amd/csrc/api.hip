@@ -79,6 +79,14 @@ static void launch_decode_exact(int g, dim3 grid, const tri::DecodeArgs& d, hipS
   }
 }
 
+// Whether a decode call reads its task table.  With exact heads only if n_tasks is negative (minus the listed
+// splits): n_tasks >= 0 promises nothing about the exact heads' splits or about the partials of splits left out, so
+// such a call gathers from the metadata rows.  So does a growing cache with exact heads, whose growth splits have no
+// task rows.
+static bool reads_tasks(const void* tasks, int n_tasks, const int32_t* xslot, const int64_t* tail_base) {
+  return tasks != nullptr && (xslot == nullptr || (n_tasks < 0 && tail_base == nullptr));
+}
+
 // CU count of the current device, cached per device (devices 0..63)
 static int device_cus(int* cus) {
   static std::atomic<int> cached[64];
@@ -428,8 +436,9 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
   d.maxn = maxn;
   d.per = per;
   d.bounds = bounds;
-  d.tasks = static_cast<const int32_t*>(tasks);  // (lists the splits to run)
-  if (d.tasks && (n_tasks < 1 || !aligned(tasks, 16))) return fail("decode: a task table needs n_tasks >= 1, 16-byte aligned");
+  d.tasks = reads_tasks(tasks, n_tasks, xslot, tail_base) ? static_cast<const int32_t*>(tasks) : nullptr;
+  const int64_t listed = xslot ? -(int64_t)n_tasks : n_tasks;
+  if (d.tasks && (listed < 1 || !aligned(tasks, 16))) return fail("decode: a task table needs n_tasks >= 1, 16-byte aligned");
   d.tiles_max = tiles_max;
   d.splits = splits;
   d.total = (int64_t)splits * hk * batch;
@@ -445,8 +454,8 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
     //   XCD step 8 * scatter mod L is the integer nearest 0.618 L coprime with L.
     const int64_t all = (int64_t)splits * hk * batch;
     if (all >= ((int64_t)1 << 31) - 1) return fail("decode: too many splits x heads x sequences");
-    if (d.tasks && n_tasks > all) return fail("decode: the task table lists more splits than exist");
-    const int64_t items = d.tasks ? n_tasks : all;
+    if (d.tasks && listed > all) return fail("decode: the task table lists more splits than exist");
+    const int64_t items = d.tasks ? listed : all;
     const bool pinned = bounds == nullptr && items % 8 == 0 && splits % 2 == 0;
     if (d.tasks) {
       // a task table lists its splits in the order to run them (costliest first): workgroup lin takes
@@ -660,7 +669,7 @@ int tri_decode_noalloc(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
   float* pm = s;
   float* pl = s + pad;
   float* po = s + 2 * pad;
-  if (tasks) {
+  if (reads_tasks(tasks, n_tasks, xslot, tail_base)) {
     // splits a task table leaves out are never written: the scratch (which holds whatever the last
     // call left) gets the empty partial in every slot first
     tri::fill_empty_partials_kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, hs>>>(pm, pl, po, n);

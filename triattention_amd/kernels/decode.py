@@ -592,7 +592,7 @@ class DecodeCache:
                 e["v"][I8], e["v"][I4], e["vstat"], e["kstat"], e["tail_k"], e["tail_v"], k, k, self.step, out,
                 *e[("partials", hq)], e["prompt"], e["per"], scale, e["xslot"], e["kx"], e["vx"], e["bounds"],
                 e.get("tasks") if self.tasks else None,
-                tail_base=e["store"].arrays["tail_base"] if e["grow_splits"] else None)
+                tail_base=e["store"].arrays["tail_base"] if e["grow_splits"] else None, exact_tasks=True)
         return e[key]
 
     def _spill_plan(self, e):

@@ -322,12 +322,13 @@ class Module:
 
     def plan_decode(self, q, k8c, k4c, ka, ka4, entry, kinfo, count, fmt, slot, v8, v4, vstat, kstat, ktail, vtail,
                     kcur, vcur, step, out, pm, pl, po, prompt, per, scale, xslot=None, kxc=None, vxc=None,
-                    bounds=None, tasks=None, tail_base=None):
+                    bounds=None, tasks=None, tail_base=None, exact_tasks=False):
         """Validate and marshal every argument of ``decode`` once (extension).  The returned
         plan's ``run(q, kcur, vcur, out, phase)`` launches with new q / k / v / out tensors of the
         planned shapes and strides and the same cache, at a few microseconds of host time.
         ``tasks``: (table, listed splits) as ``decode_tasks`` returns it for this cache and split, or None;
-        the caller keeps the partials of the splits it leaves out empty.  ``tail_base``: the int64
+        the caller keeps the partials of the splits it leaves out empty; with ``xslot`` it is ignored unless
+        ``exact_tasks`` says that it lists the exact heads' splits too.  ``tail_base``: the int64
         tokens ``tail_spill`` has moved from the tail into the cache (the tail then holds step - tail_base
         tokens), or None for the reference's tail."""
         _check(q.dtype == torch.bfloat16 and q.dim() == 4 and q.size(2) == 1 and q.size(3) == D and q.stride(3) == 1,
@@ -406,7 +407,8 @@ class Module:
                 _ptr(pl), _ptr(po), _ptr(prompt_t), b, hq, hk, maxn, int(per), tiles_max, k8c.size(0),
                 0 if k4c is None else k4c.size(0), v8.size(0), v4.size(0), _ptr(xslot), _ptr(kxc),
                 _ptr(vxc), 0 if kxc is None else kxc.numel() * kxc.element_size() // KX_BYTES, _ptr(bounds),
-                splits if bounds is not None else 0, _ptr(table), int(n_tasks), _ptr(tail_base), float(scale), 0]
+                splits if bounds is not None else 0, _ptr(table),
+                -int(n_tasks) if exact_tasks and xslot is not None else int(n_tasks), _ptr(tail_base), float(scale), 0]
         keep = (k8c, k4c, ka, ka4, entry, kinfo, count, fmt, slot, v8, v4, vstat, kstat, ktail, vtail, step, pm, pl,
                 po, prompt_t, xslot, kxc, vxc, bounds, table, tail_base)
         return DecodePlan(self, args, q, kcur, out, keep)
