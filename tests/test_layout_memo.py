@@ -58,3 +58,25 @@ def test_layouts_are_bounded():
         store(cache, 0, 64 * tiles)
     assert len(cache.layouts) == 3
     assert store(cache, 0, 64)["splits"] >= 1 and len(cache.layouts) == 3
+
+
+@pytest.mark.gpu
+def test_layouts_are_shared_within_one_stream(module):
+    from helpers import bands_fn_of
+    from triattention_amd.kernels.prefill import Prefill
+
+    cache = DecodeCache(module, max_tail=8)
+    pre = Prefill(module, bands_fn_of(BANDS), cache)
+    kv = torch.ones(1, 2, 200, 128, device="cuda", dtype=torch.bfloat16)
+    q = torch.ones(1, 4, 1, 128, device="cuda", dtype=torch.bfloat16)
+    other = torch.cuda.Stream()
+    layouts, outs = [], []
+    for stream in (None, None, other, other):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            pre.store_only(0, kv, kv, 4)
+            outs.append(cache(0, q, kv[:, :, :1].contiguous(), kv[:, :, :1].contiguous(), 0.1))
+        layouts.append(cache.layers[0]["layout"])
+    torch.cuda.synchronize()
+    assert layouts[0] is layouts[1] and layouts[2] is layouts[3] and layouts[0] is not layouts[2]
+    assert all(torch.equal(outs[0], o) for o in outs)

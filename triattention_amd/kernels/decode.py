@@ -177,6 +177,11 @@ def balanced_partition(metas, batches, slots: int):
     return [torch.from_numpy(pad(b).astype(np.int32)) for b in out], splits
 
 
+def _stream(device):
+    """(device, its current stream's handle): what a shared device tensor belongs to."""
+    return device, torch.cuda.current_stream(device).cuda_stream if device.type == "cuda" else 0
+
+
 class _LayerStore:
     """A layer's decode-cache arrays on the device, with room to append sequences: per-sequence rows
     (metadata [rows][hk][maxn], scales [rows][hk][tiles_max][4], statistics, bf16 tails) and the
@@ -406,7 +411,8 @@ class DecodeCache:
         """The split partition over every stored group (host metadata, no device sync): per, splits, bounds on
         the host and the device, and room for the task items that ``plan`` derives from them.  It depends on
         lengths, bands and the wave alone, so every prompt of one shape (each layer of a model, each new
-        prompt) shares it; ragged batches of several stores compute their own."""
+        prompt) shares it; ragged batches of several stores compute their own.  Each stream has layouts of its
+        own: their device tensors go back to the stream they were made on."""
         if self.wave is None:
             cus = self.module.device_cus() if hasattr(self.module, "device_cus") else \
                 torch.cuda.get_device_properties(st.device).multi_processor_count
@@ -414,7 +420,7 @@ class DecodeCache:
         if len(st.groups) > 1:
             return self._partition(st)
         g = st.groups[0]
-        key = (g["meta"]["key"], g["batch"], st.maxn, st.grow_tiles, self.per, self.wave)
+        key = (g["meta"]["key"], g["batch"], st.maxn, st.grow_tiles, self.per, self.wave, _stream(st.device))
         hit = self.layouts.pop(key, None)
         if hit is None:
             hit = self._partition(st)
@@ -571,10 +577,11 @@ class DecodeCache:
             if self.tasks and "tasks" not in e and hasattr(self.module, "decode_tasks") and \
                     (e["xslot"] is None or not e["grow_splits"]):
                 layout = e["layout"]
-                if "items" not in layout:
+                key_items = "items", _stream(q.device)
+                if key_items not in layout:
                     items_host = self._task_items(e)
-                    layout["items"] = items_host, torch.from_numpy(items_host).to(q.device)
-                items_host, items = layout["items"]
+                    layout[key_items] = items_host, torch.from_numpy(items_host).to(q.device)
+                items_host, items = layout[key_items]
                 e["tasks"] = self.module.decode_tasks(e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"],
                                                       e["slot"], e["per"], e["bounds"], items)
                 if e["grow_splits"]:
