@@ -129,6 +129,9 @@ class Module:
 
     def _launch(self, device, fn, *args):
         """``fn(*args, stream)`` on ``device``'s current stream, with that device current."""
+        # (a host tensor's device has no index either: its address must not reach a kernel)
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
         index = device.index if device.index is not None else torch.cuda.current_device()
         stream = torch.cuda.current_stream(index).cuda_stream
         if torch.cuda.current_device() == index:
