@@ -9,9 +9,12 @@ import types
 import pytest
 import torch
 
-from triattention_amd.kernels.extension import KX_BYTES, STAT_BLOCKS, Module
+from helpers import bands_fn_of
+from triattention_amd import synthetic as S
+from triattention_amd.kernels.extension import KX_BYTES, Module
+from triattention_amd.kernels.prefill import Prefill
 
-GPU = torch.device("cuda", 0)
+GPU, OTHER = torch.device("cuda", 0), torch.device("cuda", 1)
 
 
 class OnGpu(torch.Tensor):
@@ -19,6 +22,11 @@ class OnGpu(torch.Tensor):
     __torch_function__ = torch._C._disabled_torch_function_impl
     is_cuda = property(lambda self: True)
     device = property(lambda self: GPU)
+
+
+class OnOther(OnGpu):
+    """The same on another GPU."""
+    device = property(lambda self: OTHER)
 
 
 class Recorder:
@@ -90,3 +98,29 @@ def test_host_tensors_are_refused(module, monkeypatch, entry):
     monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: empty(*a, **kw))
     entry(module, gpu)
     assert len(module.lib.calls) == 1
+
+
+@pytest.mark.parametrize("exact", [[], [1], [0, 1]])
+@pytest.mark.parametrize("place", [lambda t: t, lambda t: t.as_subclass(OnOther)])
+@pytest.mark.parametrize("which", ["k", "v"])
+def test_a_prompt_on_two_devices_is_refused(module, monkeypatch, exact, place, which):
+    """Q, K and V go to one launch as raw addresses, whatever the map keeps quantized or exact."""
+    empty, to = torch.empty, torch.Tensor.to
+    monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: empty(*a, **kw))
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, d, *a: gpu(t) if d == GPU else to(t, d, *a))
+    x = lambda h: torch.zeros(1, h, 70, 128, dtype=torch.bfloat16)
+    qkv = dict(q=gpu(x(4)), k=gpu(x(2)), v=gpu(x(2)))
+    bands = torch.tensor([[S.INF, S.INF], [1, S.INF], [S.INF, S.INF], [1, S.INF]], dtype=torch.int32)
+    prefill = Prefill(module, bands_fn_of(bands, exact))
+    with pytest.raises(RuntimeError, match="on one device|BF16 V"):
+        prefill(0, **dict(qkv, **{which: place(x(2))}), scale=0.1)
+    assert module.lib.calls == []
+    with pytest.raises(RuntimeError, match="on one device"):
+        rec = gpu(torch.zeros(4 * KX_BYTES, dtype=torch.uint8))
+        kv = {n: qkv[n] for n in "kv"}
+        module.pack_exact(**dict(kv, **{which: place(x(2))}), exact=gpu(i32(4)), nx=1, kx=rec, vx=rec)
+    assert module.lib.calls == []
+    # on one device the prompt is prepared (its attention then finds the stand-in scratch on the host)
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        prefill(0, **qkv, scale=0.1)
+    assert module.lib.calls == ["tri_pack_exact" if len(exact) == 2 else "tri_prepare"]
