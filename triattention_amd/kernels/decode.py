@@ -511,6 +511,7 @@ class DecodeCache:
     def __call__(self, layer, q, k, v, scale):
         e = self._grow_step(layer)
         st = e["store"]
+        scale = float(scale)  # (a plan holds the number; a tensor's or array's may change in place)
         dtype = self.out_dtype or q.dtype
         out = torch.empty(q.shape, dtype=dtype, device=q.device)
         # the plan by the raw shapes and strides of this call's tensors (``out`` is contiguous): ``plan`` and
