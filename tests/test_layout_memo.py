@@ -60,6 +60,19 @@ def test_layouts_are_bounded():
     assert store(cache, 0, 64)["splits"] >= 1 and len(cache.layouts) == 3
 
 
+def test_growth_turned_on_later_leaves_earlier_sequences_without_room(monkeypatch):
+    """tail_spill follows a row's growth regions wherever its first word is not negative."""
+    # (77: what an unwritten allocation may hold)
+    monkeypatch.setattr(torch, "empty", lambda shape, dtype, **kw: torch.zeros(shape, dtype=dtype).fill_(77)
+                        if dtype != torch.uint32 else torch.zeros(shape, dtype=dtype))
+    cache = DecodeCache(HostCacheModule(), max_tail=64)
+    store(cache, 0, 200)
+    cache.ragged, cache.grow_tail = True, 128
+    store(cache, 0, 130)
+    grow = cache.layers[0]["store"].arrays["grow"]
+    assert bool((grow[0] == -1).all()) and bool((grow[1, :, 0] >= 0).all())
+
+
 @pytest.mark.gpu
 def test_layouts_are_shared_within_one_stream(module):
     from helpers import bands_fn_of

@@ -252,8 +252,10 @@ class _LayerStore:
                 self.tail_clear = True
             for name in ("tail_k", "tail_v"):
                 self._regrow(name, tail, 0.0, torch.bfloat16)
-            self._regrow("grow", (cap_rows, hk, 4), -1, i32, whole and not self.grow_tiles)
             self._regrow("count0", (cap_rows, hk), 0, i32, whole)
+        if self.grow_tiles and (relayout or self.arrays["grow"] is None):
+            # (rows of sequences stored without growth room hold -1: no tile of theirs is taken)
+            self._regrow("grow", (cap_rows, hk, 4), -1, i32)
         if (int4 or self.arrays["ka4"] is not None) and (relayout or self.arrays["ka4"] is None):
             self._regrow("ka4", (cap_rows, hk, tiles_max, 4), 1.0, f32, whole)
         if (exact or self.arrays["xslot"] is not None) and (relayout or self.arrays["xslot"] is None):
