@@ -60,6 +60,21 @@ def test_layouts_are_bounded():
     assert store(cache, 0, 64)["splits"] >= 1 and len(cache.layouts) == 3
 
 
+def test_layouts_are_dropped_under_another_threads_feet():
+    """Two stores that drop the same layout: the second finds it gone, or the dict changed while it looked."""
+    class Racing(dict):
+        def __iter__(self):
+            for key in list(dict.__iter__(self)):
+                dict.pop(self, key, None)  # the other thread's drop, between finding a key and dropping it
+                yield key
+
+    cache = DecodeCache(HostCacheModule(), max_tail=8)
+    cache.LAYOUTS = 1
+    store(cache, 0, 64)
+    cache.layouts = Racing(cache.layouts)
+    store(cache, 0, 128)
+
+
 def test_growth_turned_on_later_leaves_earlier_sequences_without_room(monkeypatch):
     """tail_spill follows a row's growth regions wherever its first word is not negative."""
     # (77: what an unwritten allocation may hold)

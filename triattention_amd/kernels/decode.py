@@ -427,8 +427,9 @@ class DecodeCache:
         if hit is None:
             hit = self._partition(st)
         self.layouts[key] = hit  # most recently used last
-        while len(self.layouts) > self.LAYOUTS:
-            self.layouts.pop(next(iter(self.layouts)))
+        # (threads that store at once may drop the same ones)
+        for old in list(self.layouts)[:-self.LAYOUTS]:
+            self.layouts.pop(old, None)
         return hit
 
     def _partition(self, st):
