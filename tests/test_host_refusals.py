@@ -81,8 +81,8 @@ def cache_store(module, wrap):
     row = lambda *s, dtype=torch.int32: wrap(torch.zeros(1, 2, *s, dtype=dtype))
     stat = lambda: row(3, 128, dtype=torch.float32)
     dst = dict(entry=row(1), kinfo=row(1), slot=row(1), count=row(), fmt=wrap(i32(1, 1)), prompt=wrap(i32(1)),
-               xslot=None, ka=row(1, 4, dtype=torch.float32), ka4=None, kstat=stat(), vstat=stat(), k8=rec(2048), k4=None,
-               v8=rec(2048), v4=None, kx=None, vx=None)
+               xslot=None, ka=row(1, 4, dtype=torch.float32), ka4=None, kstat=stat(), vstat=stat(), k8=rec(2048),
+               k4=None, v8=rec(2048), v4=None, kx=None, vx=None)
     zero = dict(k8=0, k4=0, v8=0, v4=0, x=0)
     module.cache_store(gpu(i32(4, 2)), None, 64, rec(2048), None, row(1, 4, dtype=torch.float32), None, stat(), stat(),
                        rec(2048), None, None, None, 0, 0, dst, zero, dict(zero, k8=2, v8=2))

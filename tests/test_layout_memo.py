@@ -6,7 +6,8 @@ import pytest
 import torch
 
 from cache_host import HostCacheModule
-from triattention_amd.kernels.decode import DecodeCache
+from triattention_amd.kernels.decode import DecodeCache, balanced_partition, entry_costs, sequence_metadata, \
+    split_bounds
 from triattention_amd.kernels.prefill import F16, I4, I8
 from triattention_amd.synthetic import INF
 
@@ -49,6 +50,41 @@ def test_a_shared_layout_equals_a_fresh_one(prompt, batch):
     assert again["per"] == fresh["per"] and again["splits"] == fresh["splits"]
     assert np.array_equal(again["bounds_host"], fresh["bounds_host"])
     assert np.array_equal(DecodeCache._task_items(again), DecodeCache._task_items(fresh))
+
+
+def bisected(meta, batch, slots):
+    """The partition by sixty steps of bisection over the target cost of a run, whatever the cache's size."""
+    costs, count = entry_costs(meta), meta["count"].numpy()
+    heads, floor = costs.sum(1), np.maximum((count + 63) // 64, 1)
+    runs = lambda t: np.maximum(np.minimum(np.ceil(heads / t), count), floor)
+    lo, hi = float(costs[costs > 0].min()), float(heads.max()) + 1
+    if batch * runs(hi).sum() <= slots:
+        for _ in range(60):
+            mid = (lo + hi) / 2
+            lo, hi = (lo, mid) if batch * runs(mid).sum() <= slots else (mid, hi)
+    n = runs(hi).astype(np.int64)
+    while True:
+        b = split_bounds(costs, meta["valid"].numpy(), n)
+        if (np.diff(b, axis=1) <= 64).all():
+            return b
+        n = n + (np.diff(b, axis=1) > 64).any(1)
+
+
+@pytest.mark.parametrize("tiles, batch, exact", [
+    (1, 1, []), (1, 5, [0]), (33, 1, [1]), (64, 1, []), (64, 4, [0, 1]), (64, 9, [0]), (256, 2, [1]), (511, 2, []),
+    (2048, 1, [0]), (300, 9, [])])
+@pytest.mark.parametrize("slots", [8, 1024])
+def test_a_short_cache_is_cut_without_bisection(monkeypatch, tiles, batch, exact, slots):
+    """A cache whose every run may be one tile is cut in one evaluation, to the bounds that bisection gives (a new
+    prompt length pays for this on the host)."""
+    codes = DecodeCache(HostCacheModule()).codes(tiles)[0]
+    meta = sequence_metadata(BANDS, tiles, 2, codes, exact)
+    want = bisected(meta, batch, slots)
+    evaluations, ceil = [], np.ceil
+    monkeypatch.setattr(np, "ceil", lambda x: evaluations.append(1) or ceil(x))
+    (got,), splits = balanced_partition([meta], [batch], slots)
+    assert splits == want.shape[1] - 1 and np.array_equal(got.numpy(), want)
+    assert len(evaluations) <= (2 if batch * int(meta["count"].sum()) <= slots else 63)
 
 
 def test_layouts_are_bounded():
