@@ -1,7 +1,9 @@
 """GPU parity of the two prepare launches (tri_prepare_qk, tri_pack_v, tri_pack_exact, tri_prepare).
 
 Codes, scales, statistics and records are whole numbers or single correctly rounded operations: every
-array is held to the oracle bit for bit, and the one-call form to the three separate calls.  Sizes: one
+array is held to the oracle bit for bit at every size, the expanded INT4 keys and the V8 sums to the records
+they come from, the exact heads' records to a host packing of the documented layout, and the one-call form to
+the three separate calls.  The bytes past each buffer stay as they were.  Sizes: one
 token, either side of a tile, prompts whose record workgroups take one tile each and several (a head's
 last workgroup then takes fewer), statistics chains of one load batch, two and a remainder; inputs
 token-major (as HF projections give them), head-major, and a padded row stride.
@@ -13,13 +15,17 @@ import pytest
 import torch
 
 import oracle as O
+from cache_host import pack_kx
 from helpers import compare_codes
 from triattention_amd import synthetic as S
+from triattention_amd.kernels import records as R
 from triattention_amd.kernels.prefill import F16, I4, I8, Layout, Prefill, Q4
 from triattention_amd.maps import uniform
 from triattention_amd.synthetic import bits
 
 pytestmark = pytest.mark.gpu
+
+GUARD, FILL = 4096, 0xA5  # bytes past each buffer, and what every byte holds before the calls
 
 
 def on_device(x, layout):
@@ -33,6 +39,31 @@ def on_device(x, layout):
     return y[..., :d].transpose(1, 2)
 
 
+def guarded(module, lay, device):
+    """A prompt's operands in a scratch of their sizes plus GUARD bytes, every byte FILL; and a check that
+    those bytes still are."""
+    sizes, pre = Prefill(module, uniform(1, 2)), Prefill(module, uniform(1, 2))
+    sizes.operands(lay, device)
+    for name, x in sizes.buffers.items():
+        pool = torch.full((x.numel() * x.element_size() + GUARD,), FILL, dtype=torch.uint8, device=device)
+        pre.buffers[name] = pool.view(x.dtype)
+
+    def check():
+        for name, x in pre.buffers.items():
+            n = sizes.buffers[name].numel() * x.element_size()
+            assert bool((x.view(torch.uint8)[n:] == FILL).all()), f"written past {name}"
+    return pre.operands(lay, device), check
+
+
+def all_codes(q, k, v):
+    """The oracle's operands of one sequence with every format, whatever a map of this length would keep."""
+    _, kstat = O.stats(k)
+    _, vstat = O.stats(v)
+    names = ("q8", "qa", "q4", "qa4", "k8", "ka", "k4", "ka4", "v16", "v8", "v4")
+    codes = dict(zip(names, O.quantize_q(q, True) + O.quantize_k(k, kstat, True) + O.pack_v(v, vstat)))
+    return dict(codes, kstat=kstat, vstat=vstat)
+
+
 @pytest.mark.parametrize("batch, hq, hk, t, layout", [
     (1, 6, 2, 1, "head"), (2, 3, 3, 64, "token"), (1, 4, 2, 65, "padded"), (1, 2, 1, 1025, "token"),
     (2, 4, 4, 8193, "head"), (3, 8, 8, 3001, "padded")])
@@ -42,11 +73,7 @@ def test_prepare_matches_the_oracle_and_the_separate_calls(module, batch, hq, hk
     host = [S.outlier_tensor(g, batch, h, t) for h in (hq, hk, hk)]
     q, k, v = (on_device(x, layout) for x in host)
     lay = Layout(batch, hq, hk, t, True, frozenset((F16, I8, I4, Q4)))
-    pres = [Prefill(module, uniform(1, 2)) for _ in range(2)]
-    ops, sep = (p.operands(lay, q.device) for p in pres)
-    for x in list(ops.values()) + list(ops["packed"].values()) + list(sep.values()) + list(sep["packed"].values()):
-        if isinstance(x, torch.Tensor):
-            x.view(torch.uint8).fill_(0xA5)
+    (ops, past), (sep, past_sep) = (guarded(module, lay, q.device) for _ in range(2))
     p, s = ops["packed"], sep["packed"]
     module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"], ops["q4"],
                    ops["qa4"], ops["k4"], ops["ka4"], ops["k4x"], ops["vpartial"], ops["vstat"], p[F16], p[I8], p[I4],
@@ -59,28 +86,63 @@ def test_prepare_matches_the_oracle_and_the_separate_calls(module, batch, hq, hk
         assert torch.equal(ops[name].view(torch.uint8), sep[name].view(torch.uint8)), name
     for code in (F16, I8, I4):
         assert torch.equal(p[code].view(torch.uint8), s[code].view(torch.uint8)), code
-    bands = np.array([[1, 1 << 20]] * hq)
+    past()
+    past_sep()
+    tiles = (t + 63) // 64
+    k4x = R.unpack_k8(ops["k4x"].cpu().numpy()).reshape(batch, hk, tiles * 64, 128)
+    sums = ops["v8sum"].cpu().numpy().reshape(batch, hk, tiles, 128)
     for b in range(batch):
-        codes = O.prefill_codes(*(bits(x[b]) for x in host), bands, decode_cache=t > 1088)
-        if codes["v4"] is None:  # (short prompts keep no INT4 V: pack it from the same statistics)
-            codes["v4"] = O.pack_v(bits(host[2][b]), codes["vstat"], True, True, True)[2]
-        if not codes["identity"]:
-            compare_codes(ops, codes, b, batch, hq, hk, t)
+        codes = all_codes(*(bits(x[b]) for x in host))
+        compare_codes(ops, codes, b, batch, hq, hk, t)
+        np.testing.assert_array_equal(k4x[b].astype(np.int32), 16 * codes["k4"].astype(np.int32))
+        np.testing.assert_array_equal(sums[b], -127 * codes["v8"].reshape(hk, tiles, 64, 128).sum(2, dtype=np.int32))
 
 
-@pytest.mark.parametrize("t, flags", [(1, [1, 0]), (130, [0, 1]), (130, [2, 1])])
+@pytest.mark.parametrize("t", [1, 64, 65])
+def test_prepare_without_quantized_v_keeps_it(module, t):
+    """With V16 records alone V' is V itself: the statistics are (0, 1, 1), the records V's fp16 values."""
+    g = S.gen(7050 + t)
+    host = [S.outlier_tensor(g, 2, h, t) for h in (4, 2, 2)]
+    q, k, v = (x.cuda() for x in host)
+    ops, past = guarded(module, Layout(2, 4, 2, t, False, frozenset((F16,))), q.device)
+    module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"], None, None, None,
+                   None, None, ops["vpartial"], ops["vstat"], ops["packed"][F16], None, None, None)
+    past()
+    for b in range(2):
+        codes = O.prefill_codes(*(bits(x[b]) for x in host), np.array([[9, 9]] * 4))
+        assert codes["identity"] and codes["k4"] is None and codes["v8"] is None
+        compare_codes(ops, codes, b, 2, 4, 2, t)
+
+
+@pytest.mark.parametrize("t, flags", [(1, [1, 0]), (64, [0, 1]), (65, [0, 1, 2]), (130, [0, 1]), (130, [2, 1])])
 def test_prepare_writes_the_exact_records(module, t, flags):
-    """The exact heads' KX / VX records of the one-call form equal pack_exact's; a quantized head's are
-    left alone."""
+    """The exact heads' KX / VX records of the one-call form and of pack_exact are the documented layout's,
+    zeros past the prompt; nothing is written for a quantized head, nor outside the records."""
     g = S.gen(7100 + t)
-    q, k, v = (S.outlier_tensor(g, 2, h, t).cuda() for h in (4, 2, 2))
+    batch, hk, hq = 2, len(flags), 2 * len(flags)
+    host = [S.outlier_tensor(g, batch, h, t) for h in (hq, hk, hk)]
+    q, k, v = (x.cuda() for x in host)
     tiles, nx = (t + 63) // 64, max(flags)
     exact = torch.tensor([f for f in flags for _ in range(2)], dtype=torch.int32, device="cuda")
-    pre = Prefill(module, uniform(1, 2))
-    ops = pre.operands(Layout(2, 4, 2, t, False, frozenset((F16,))), q.device)
-    out = [torch.full((2 * nx * tiles * 16384,), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    ops, past = guarded(module, Layout(batch, hq, hk, t, False, frozenset((F16,))), q.device)
+    # (a head's records of guard on either side: a quantized head has slot -1)
+    n, guard = batch * nx * tiles * 16384, tiles * 16384
+    out = [torch.full((n + 2 * guard,), FILL, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    kx, vx, kx2, vx2 = (x[guard:guard + n] for x in out)
     module.prepare(q, k, v, ops["q8"], ops["qa"], ops["kp"], ops["ka"], ops["partial"], ops["kstat"], None, None, None,
-                   None, None, ops["vpartial"], ops["vstat"], ops["packed"][F16], None, None, None, exact, nx, *out[:2])
-    module.pack_exact(k, v, exact, nx, *out[2:])
-    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+                   None, None, ops["vpartial"], ops["vstat"], ops["packed"][F16], None, None, None, exact, nx, kx, vx)
+    module.pack_exact(k, v, exact, nx, kx2, vx2)
+    past()
+    want = np.zeros((2, batch, nx, tiles, 16384), np.uint8)
+    rows = np.zeros((2, batch, hk, tiles * 64, 128), np.uint16)
+    for i, x in enumerate(host[1:]):
+        rows[i, :, :, :t] = bits(x)
+    for h, f in enumerate(flags):
+        for b in range(batch if f else 0):
+            for j in range(tiles):
+                want[:, b, f - 1, j] = pack_kx(*rows[:, b, h, 64 * j:64 * j + 64])
+    for i, x in enumerate(out):
+        got = x.cpu().numpy()
+        np.testing.assert_array_equal(got[guard:guard + n], want[i % 2].reshape(-1))
+        assert (got[:guard] == FILL).all() and (got[guard + n:] == FILL).all()
     assert bool((ops["vstat"][:, :, 0] == 0).all()) and bool((ops["vstat"][:, :, 1:] == 1).all())  # identity V
