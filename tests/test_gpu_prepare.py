@@ -146,3 +146,25 @@ def test_prepare_writes_the_exact_records(module, t, flags):
         np.testing.assert_array_equal(got[guard:guard + n], want[i % 2].reshape(-1))
         assert (got[:guard] == FILL).all() and (got[guard + n:] == FILL).all()
     assert bool((ops["vstat"][:, :, 0] == 0).all()) and bool((ops["vstat"][:, :, 1:] == 1).all())  # identity V
+
+
+def test_prepare_qk_past_one_grid(module):
+    """65,535 one-token sequences of 257 q-heads: 17.9 million workgroups, more than one grid holds.  Every row
+    holds its sequence's codes, as the same sequences with one q-head in one grid give them."""
+    batch, heads = 65535, 257
+    g = torch.Generator(device="cuda").manual_seed(7200)
+    q, k = (torch.randn(batch, 1, 1, 128, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    new = lambda *shape, dtype=torch.float32: torch.full(shape, 7, dtype=dtype, device="cuda")
+    kp, partial, outs = new(batch * 2048, dtype=torch.int32), new(batch * 64 * 3 * 128), []
+    for h in (1, heads):
+        q8, qa, ka, kstat = new(batch, h, 1, 128, dtype=torch.int8), new(batch * h), new(batch * 4), new(batch * 3 * 128)
+        print(f"\n[prepare] {batch} sequences of one token, {h} q-heads", flush=True)
+        module.prepare_qk(q.expand(-1, h, -1, -1), k, q8, qa, kp.view(torch.uint32), ka, partial, kstat)
+        outs.append((q8.view(batch, h, 128), qa.view(batch, h), ka, kstat, kp.clone()))
+    one, many = outs
+    for b in range(0, batch, 4096):  # (a slice at a time: the comparison's temporaries stay small)
+        assert bool((many[0][b:b + 4096] == one[0][b:b + 4096]).all())
+    assert bool((many[1] == one[1]).all())
+    assert all(torch.equal(x, y) for x, y in zip(one[2:], many[2:]))
+    codes = O.quantize_q(bits(q[:64, 0].cpu()), False)  # [64 rows as heads, one token]
+    np.testing.assert_array_equal(one[0][:64, 0].cpu().numpy(), codes[0][:, 0])

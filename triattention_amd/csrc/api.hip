@@ -202,6 +202,11 @@ static int pack_exact_args(tri::PrepareArgs& a, const void* k, int64_t k_sb, int
   return 0;
 }
 
+// Workgroups per launch of a prepare kernel.  A grid dimension holds fewer than 2^32 threads (2^24 workgroups of 256):
+// past that the runtime reports no error and runs only the remainder (measured at 17.9 million workgroups).  The
+// statistics of 524,288 (sequence, KV head) pairs, or the Q codes of 2^24 short rows, reach it; such calls go in several launches.
+constexpr int64_t PREPARE_GRID = 1 << 23;
+
 // The launches of the parts that are present (k8, v16 / v8 / v4 with vstat, exact).
 static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) {
   const int64_t tiles = (a.t + tri::BN - 1) / tri::BN, heads = (int64_t)a.hk * a.batch;
@@ -221,8 +226,14 @@ static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) 
   a.vstat_wgs = has_v && !a.v_identity ? (int)stat : 0;
   a.krec_wgs = has_k ? (int)rec : 0;
   a.vrec_wgs = has_v ? (int)rec : 0;
-  if (g1 > 0) tri::prepare_stats_kernel<<<dim3((unsigned)g1), 256, 0, s>>>(a);
-  tri::prepare_records_kernel<<<dim3((unsigned)g2), 256, 0, s>>>(a);
+  for (int64_t w = 0; w < g1; w += PREPARE_GRID) {
+    a.wg0 = (int)w;
+    tri::prepare_stats_kernel<<<dim3((unsigned)std::min(PREPARE_GRID, g1 - w)), 256, 0, s>>>(a);
+  }
+  for (int64_t w = 0; w < g2; w += PREPARE_GRID) {
+    a.wg0 = (int)w;
+    tri::prepare_records_kernel<<<dim3((unsigned)std::min(PREPARE_GRID, g2 - w)), 256, 0, s>>>(a);
+  }
   return check_launch(what);
 }
 

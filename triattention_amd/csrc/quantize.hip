@@ -36,8 +36,8 @@ struct PrepareArgs {
   const int32_t* exact;    // [hq]: 1 + record slot of the q-head's KV head, 0 if quantized
   int nx;
   uint8_t *kx, *vx;
-  // workgroups per part and tiles per record workgroup (set by the host)
-  int kstat_wgs, vstat_wgs, krec_wgs, vrec_wgs, per, chunks;
+  // workgroups per part, tiles per record workgroup, and the launch's first workgroup (set by the host)
+  int kstat_wgs, vstat_wgs, krec_wgs, vrec_wgs, per, chunks, wg0;
 };
 
 // Q codes: one 128-feature row per 8 lanes (16 features per lane, rotated with DPP lane moves by
@@ -136,7 +136,7 @@ __device__ __forceinline__ void stat_block(const uint16_t* __restrict__ src, int
 // (Q codes, K partials, V partials): 4 x 8192 tokens, Hq 28 / Hk 4, 111 -> 105 us (4.6 TB/s, a plain copy
 // reaches 4.85); 30,001 tokens, Hq 32 / Hk 8, 163 -> 109 us; 1,024 tokens, Hq 24 / Hk 8, 14 -> 7.8 us.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void prepare_stats_kernel(PrepareArgs a) {
-  int wg = blockIdx.x;
+  int wg = a.wg0 + blockIdx.x;
   if (wg < a.kstat_wgs + a.vstat_wgs) {
     const bool isv = wg >= a.kstat_wgs;
     if (isv) wg -= a.kstat_wgs;
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(256) void prepare_records_kernel(PrepareArgs a) {
   __shared__ int vsum[D];
   static_assert(sizeof(stage) >= 2 * BN * D && sizeof(stage) >= BN * EXACT_VP * 2, "staging");
   const int tiles = (a.t + BN - 1) / BN;
-  int wg = blockIdx.x;
+  int wg = a.wg0 + blockIdx.x;
   if (wg < a.krec_wgs) {
     const int hb = wg / a.chunks, j0 = (wg % a.chunks) * a.per, j1 = min(tiles, j0 + a.per);
     const int hd = hb % a.hk, b = hb / a.hk;
