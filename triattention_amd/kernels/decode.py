@@ -185,6 +185,11 @@ def _stream(device):
     return device, torch.cuda.current_stream(device).cuda_stream if device.type == "cuda" else 0
 
 
+def _capturing(device):
+    """Whether launches on ``device``'s current stream are being recorded into a graph instead of run."""
+    return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 class _LayerStore:
     """A layer's decode-cache arrays on the device, with room to append sequences: per-sequence rows
     (metadata [rows][hk][maxn], scales [rows][hk][tiles_max][4], statistics, bf16 tails) and the
@@ -535,7 +540,8 @@ class DecodeCache:
             plan.launch(q, k, v, out, short_tail=short)
         else:
             plan.run(q, k, v, out, short_tail=short)
-            e["calls"][shapes] = plan
+            if not _capturing(q.device):  # (see plan)
+                e["calls"][shapes] = plan
         return out
 
     # the merge runs as one wave per (sequence, q-head) while the tail holds at most SHORT_TAIL tokens on a
@@ -570,44 +576,61 @@ class DecodeCache:
     def plan(self, layer, q, k, out, scale):
         """The layer's validated decode call for q / k (and v) / out of these shapes (built once, then reused)."""
         e = self.layers[layer]
-        key = ("partials", q.shape[1])
-        if key not in e:
-            # every slot starts as the empty partial: splits that hold no kept tile are left out of the
-            # launch (the task table lists the others) and keep it
-            n = e["batch"] * q.shape[1] * e["splits"]
-            e[key] = (torch.full((n,), -3.4028234663852886e38, device=q.device), torch.zeros(n, device=q.device),
-                      torch.zeros(n * 128, device=q.device))
         key = ("plan", _geometry(q), _geometry(k), _geometry(out), float(scale))
         if key not in e:
-            hq = q.shape[1]
             # (a growing cache with exact heads gathers: tail_spill keeps no task rows for exact heads)
-            if self.tasks and "tasks" not in e and hasattr(self.module, "decode_tasks") and \
-                    (e["xslot"] is None or not e["grow_splits"]):
-                layout = e["layout"]
-                key_items = "items", _stream(q.device)
-                if key_items not in layout:
-                    items_host = self._task_items(e)
-                    layout[key_items] = items_host, torch.from_numpy(items_host).to(q.device)
-                items_host, items = layout[key_items]
-                e["tasks"] = self.module.decode_tasks(e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"],
-                                                      e["slot"], e["per"], e["bounds"], items)
-                if e["grow_splits"]:
-                    # task row of each head's first growth split (a head's growth splits are empty at the
-                    # store, so they are listed last, consecutively, in item order)
-                    first = np.arange(e["batch"] * e["store"].hk, dtype=np.int64) * e["splits"] + \
-                        (e["splits"] - e["grow_splits"])
-                    where = np.full(int(items_host.max()) + 1, -1, np.int64)
-                    where[items_host] = np.arange(items_host.size)
-                    rows = where[first].astype(np.int32)
-                    e["store"].arrays["grow"][:e["batch"], :, 3].copy_(
-                        torch.from_numpy(rows.reshape(e["batch"], e["store"].hk)))
-            e[key] = self.module.plan_decode(
-                q, e["k8"], e["k4"], e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"], e["slot"],
-                e["v"][I8], e["v"][I4], e["vstat"], e["kstat"], e["tail_k"], e["tail_v"], k, k, self.step, out,
-                *e[("partials", hq)], e["prompt"], e["per"], scale, e["xslot"], e["kx"], e["vx"], e["bounds"],
-                e.get("tasks") if self.tasks else None,
-                tail_base=e["store"].arrays["tail_base"] if e["grow_splits"] else None, exact_tasks=True)
+            tasks = self.tasks and hasattr(self.module, "decode_tasks") and (e["xslot"] is None or not e["grow_splits"])
+            if tasks and "tasks" not in e and _capturing(q.device):
+                # The table and the empty partials are filled once, now: recorded launches would leave them unfilled
+                # for the eager steps before the first replay.  A first step captured on a cache with exact heads
+                # gathers, with partials of the graph's own (every split writes its own), and is not kept.
+                if e["xslot"] is None:
+                    raise RuntimeError(f"decode cache layer {layer}: run one step before capturing one (the split "
+                                       "kernel's task table cannot be built under capture)")
+                return self._plan_decode(e, q, k, out, scale, self._partials(e, q), None)
+            hq = q.shape[1]
+            if ("partials", hq) not in e:
+                e[("partials", hq)] = self._partials(e, q)
+            if tasks and "tasks" not in e:
+                self._build_tasks(e, q.device)
+            e[key] = self._plan_decode(e, q, k, out, scale, e[("partials", hq)], e.get("tasks") if self.tasks else None)
         return e[key]
+
+    @staticmethod
+    def _partials(e, q):
+        """Split partials (m, l, o), every slot the empty partial: splits that hold no kept tile are left out of
+        the launch (the task table lists the others) and keep it."""
+        n = e["batch"] * q.shape[1] * e["splits"]
+        return (torch.full((n,), -3.4028234663852886e38, device=q.device), torch.zeros(n, device=q.device),
+                torch.zeros(n * 128, device=q.device))
+
+    def _build_tasks(self, e, device):
+        """The split kernel's task table of a layer entry (e["tasks"])."""
+        layout = e["layout"]
+        key_items = "items", _stream(device)
+        if key_items not in layout:
+            items_host = self._task_items(e)
+            layout[key_items] = items_host, torch.from_numpy(items_host).to(device)
+        items_host, items = layout[key_items]
+        e["tasks"] = self.module.decode_tasks(e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"],
+                                              e["slot"], e["per"], e["bounds"], items)
+        if e["grow_splits"]:
+            # task row of each head's first growth split (a head's growth splits are empty at the
+            # store, so they are listed last, consecutively, in item order)
+            first = np.arange(e["batch"] * e["store"].hk, dtype=np.int64) * e["splits"] + \
+                (e["splits"] - e["grow_splits"])
+            where = np.full(int(items_host.max()) + 1, -1, np.int64)
+            where[items_host] = np.arange(items_host.size)
+            rows = where[first].astype(np.int32)
+            e["store"].arrays["grow"][:e["batch"], :, 3].copy_(
+                torch.from_numpy(rows.reshape(e["batch"], e["store"].hk)))
+
+    def _plan_decode(self, e, q, k, out, scale, partials, tasks):
+        return self.module.plan_decode(
+            q, e["k8"], e["k4"], e["ka"], e["ka4"], e["entry"], e["kinfo"], e["count"], e["fmt"], e["slot"],
+            e["v"][I8], e["v"][I4], e["vstat"], e["kstat"], e["tail_k"], e["tail_v"], k, k, self.step, out,
+            *partials, e["prompt"], e["per"], scale, e["xslot"], e["kx"], e["vx"], e["bounds"], tasks,
+            tail_base=e["store"].arrays["tail_base"] if e["grow_splits"] else None, exact_tasks=True)
 
     def _spill_plan(self, e):
         """The layer's tail_spill launch (tail growth), built once per cache layout."""
