@@ -23,6 +23,9 @@ class OnGpu(torch.Tensor):
     is_cuda = property(lambda self: True)
     device = property(lambda self: GPU)
 
+    def get_device(self):
+        return self.device.index
+
 
 class OnOther(OnGpu):
     """The same on another GPU."""

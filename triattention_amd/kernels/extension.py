@@ -129,10 +129,12 @@ class Module:
 
     def _launch(self, device, fn, *args):
         """``fn(*args, stream)`` on ``device``'s current stream, with that device current."""
-        # (a host tensor's device has no index either: its address must not reach a kernel)
-        if device.type != "cuda":
-            raise ValueError(f"Expected a cuda device, but got: {device}")
-        index = device.index if device.index is not None else torch.cuda.current_device()
+        index = device.index
+        if index is None:
+            # (a host tensor's device has no index either: its address must not reach a kernel)
+            if device.type != "cuda":
+                raise ValueError(f"Expected a cuda device, but got: {device}")
+            index = torch.cuda.current_device()
         stream = torch.cuda.current_stream(index).cuda_stream
         if torch.cuda.current_device() == index:
             self._call(fn, *args, stream)
@@ -146,7 +148,7 @@ class Module:
         _check(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 4 and q.size(3) == D and q.stride(3) == 1 and
                k.dtype == torch.bfloat16 and k.dim() == 4 and k.size(0) == q.size(0) and k.size(2) == q.size(2) and
                k.size(3) == D and k.stride(3) == 1, "BF16 Q/K [B,H,T,128] with contiguous features")
-        _check(k.device == q.device, "Q/K on one device")
+        _check(k.get_device() == q.get_device(), "Q/K on one device")
 
     @staticmethod
     def _check_qk(q, k, q8, qa, kp, ka, partial, kstat, q4, qa4, k4p, ka4, k4x):
@@ -184,7 +186,7 @@ class Module:
     def _check_exact(k, v, exact, nx, kx, vx):
         _check(k.dtype == v.dtype == torch.bfloat16 and k.dim() == 4 and k.shape == v.shape and k.size(3) == D and
                k.stride(3) == 1 and v.stride(3) == 1, "K/V bf16 [B,Hk,T,128]")
-        _check(k.device == v.device, "K/V on one device")
+        _check(k.get_device() == v.get_device(), "K/V on one device")
         b, hk, t, _ = k.shape
         h = exact.numel()
         tiles = (t + 63) // 64
@@ -221,7 +223,7 @@ class Module:
         scratch buffers of their own."""
         b, hq, hk, t = self._check_qk(q, k, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x)
         _check(self._check_v(v, vpartial, vstat, v16p, v8p, v4p, v8sum) == (b, hk, t), "V [B,Hkv,T,128] like K")
-        _check(v.device == q.device, "Q/K/V on one device")
+        _check(v.get_device() == q.get_device(), "Q/K/V on one device")
         if exact is not None:
             _check(self._check_exact(k, v, exact, nx, kx, vx)[1] == hq, "exact flags [Hq]")
         self._launch(q.device, self.lib.tri_prepare, _ptr(q), *q.stride()[:3], _ptr(k), *k.stride()[:3], _ptr(v),
