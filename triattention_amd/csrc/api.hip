@@ -204,7 +204,8 @@ static int pack_exact_args(tri::PrepareArgs& a, const void* k, int64_t k_sb, int
 
 // Workgroups per launch of a prepare kernel.  A grid dimension holds fewer than 2^32 threads (2^24 workgroups of 256):
 // past that the runtime reports no error and runs only the remainder (measured at 17.9 million workgroups).  The
-// statistics of 524,288 (sequence, KV head) pairs, or the Q codes of 2^24 short rows, reach it; such calls go in several launches.
+// statistics of 524,288 (sequence, KV head) pairs, or the Q codes of 2^24 short rows, reach it; such calls go in
+// several launches.
 constexpr int64_t PREPARE_GRID = 1 << 23;
 
 // The launches of the parts that are present (k8, v16 / v8 / v4 with vstat, exact).
@@ -213,9 +214,8 @@ static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) 
   const bool has_k = a.k8 != nullptr, has_v = a.vstat != nullptr;
   const int64_t stat = heads * (tri::STAT_BLOCKS / 4);
   const int64_t qwgs = a.q8 ? (int64_t)((a.t + 31) / 32) * a.hq * a.batch : 0;
-  // Tiles per record workgroup: one while that gives at most RECORD_WGS workgroups per part (a short prompt
-  // then has a workgroup per tile), more beyond, so that the statistics each workgroup forms anew stay cheap
-  // beside its tiles.
+  // Tiles per record workgroup: one below 2 * RECORD_WGS workgroups per part (a short prompt then has a workgroup
+  // per tile), more beyond, so that the statistics each workgroup forms anew stay cheap beside its tiles.
   a.per = (int)std::max<int64_t>(1, heads * tiles / tri::RECORD_WGS);
   a.chunks = (int)((tiles + a.per - 1) / a.per);
   const int64_t rec = heads * a.chunks, xwgs = a.exact ? heads * tiles : 0;

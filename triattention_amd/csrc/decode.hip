@@ -285,7 +285,8 @@ __device__ __forceinline__ void decode_exact(const DecodeArgs& a, int b, int kh,
 // quantization and metadata, take its tiles alternately (wave w: entries first
 // + w, first + w + 2, ...), and combine their running (m, l, o) in LDS at the
 // end, so that each SIMD holds two waves whose dependency chains interleave.
-// TASKS: the launch has a task table (a.tasks), whose rows give each split's entries; a separate instantiation, so that the common path has no branch between the first
+// TASKS: the launch has a task table (a.tasks), whose rows give each split's entries; a separate
+// instantiation, so that the common path has no branch between the first
 // tile's record loads and the use of Q (at a join of two paths the compiler waits for every
 // outstanding load, which would hold the Q quantization until the records arrive).
 template <int R, bool EXACT = false, bool DUP = false, int NW = 1, int W = 2, bool TASKS = false>
@@ -867,11 +868,12 @@ struct MergeArgs {
 // (common_device.cuh:373-469).  One workgroup of NW waves per (sequence, q-head),
 // XCD-aware so the q-heads of one KV head share an L2 for their tail reads.
 // Every global load that does not depend on another is issued first (the split
-// partials of up to 64 splits, the first 32 tail tokens' K rows and first 64
-// tail tokens' V rows), so a short tail costs one memory round trip; longer
-// tails and more splits continue in loops that keep MERGE_K rounds of 32 K rows and
-// MERGE_V rounds of 16 V rows in flight.  Tail scores: 8 lanes per token (16
-// channels each); tail values: 16 lanes per token (8 channels each).
+// partials of up to 64 splits, one round of SG = 8 * NW tail tokens' K rows and
+// four of VG = 4 * NW tail tokens' V rows), so a short tail costs one memory round
+// trip; longer tails continue in loops that keep MERGE_K rounds of K rows and MERGE_V
+// rounds of V rows in flight, splits past 64 in one that takes a round trip per NW
+// of them.  Tail scores: 8 lanes per token (16 channels each); tail values: 16 lanes
+// per token (8 channels each).
 constexpr int MERGE_K = 2, MERGE_V = 4;
 // Waves per (sequence, q-head) on grids of fewer than SHORT_WIDE workgroups per CU, which leave SIMDs idle:
 // a long tail is bound by each wave's own scores and weights.  Kernel times at 4 / 8 / 16 waves: 256

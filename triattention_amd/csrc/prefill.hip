@@ -581,9 +581,9 @@ __global__ __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(2))
   // tokens 1776 -> 1762 us.)
   const int nf16 = qb > 0 ? 2 : 1;
   // this pair's part [q0, q1) of the quantized tile list (INT8 tiles, then INT4 ones): with two pairs,
-  // pair 0's F16 tiles (each priced as two quantized ones: their copies are synchronous) and quantized
-  // tiles balance pair 1's (C0 attention: 25.3 us with the F16 tiles priced as one, 23.6 as two, 24.9
-  // as three)
+  // pair 0's F16 tiles (each priced as two quantized ones) and quantized tiles balance pair 1's (C0
+  // attention: 25.3 us with the F16 tiles priced as one, 23.6 as two, 24.9 as three, all three before
+  // the diagonal's copies overlapped its scores)
   const int total = n8 + n4;
   const int c = PAIRS == 2 ? max(0, (total - 2 * nf16 + 1) / 2) : total;
   const int q0 = pair == 0 ? 0 : c, q1 = pair == 0 ? c : total;

@@ -8,7 +8,9 @@
 
 namespace tri {
 
-// Record workgroups per part (K, V) up to which each takes a single tile.  Fewer workgroups form the
+// Record workgroups per part (K, V): each takes max(1, tiles of all heads / RECORD_WGS) tiles, rounded down, so a
+// part of up to 2 * RECORD_WGS - 1 tiles has one per workgroup, and a longer one RECORD_WGS to 2 * RECORD_WGS - 1
+// workgroups (and at least one per head).  Fewer workgroups form the
 // statistics less often, more have more loads in flight (prepare_records_kernel at 256 / 512 / 1024 / 2048:
 // 4 x 8192 tokens, 4 KV heads, 46 / 41 / 46 / 52 us; 30,001 tokens, 8 KV heads, 76 / 72 / 66 / 80 us).
 constexpr int RECORD_WGS = 512;
@@ -383,7 +385,8 @@ __device__ __forceinline__ void pack_v_tile(const VRaw& in, int rows,
   }
 }
 
-// The KX / VX records of the exact KV heads.  Keys at or past t are zero.  Per 64-key tile, 16 KiB each, 32-key half kb at byte kb*8192:
+// The KX / VX records of the exact KV heads.  Keys at or past t are zero.  Per 64-key tile, 16 KiB each, 32-key
+// half kb at byte kb*8192:
 //   KX fragment F = ks (16-feature step), lane L 16 bytes = bf16 K[key kb*32 + L%32]
 //      [features ks*16 + 8*(L/32) .. +7]      (A operand of S^T = K Q^T)
 //   VX fragment F = cb*2 + kh, lane L element e = bf16 V[key kb*32 + 16*kh + 8*(e/4)

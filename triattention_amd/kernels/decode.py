@@ -144,8 +144,11 @@ def balanced_partition(metas, batches, slots: int):
     split kernel streams each split's records at about the same rate per wave, so its time is set
     by the largest split.  Heads are cut by cost (the measured time of each tile's kind) into
     n_h = min(ceil(cost_h / t), tiles) runs of near-equal cost, with the smallest target t whose split
-    count fits ``slots`` resident workgroups, at most 64 entries per split.  A short cache thus gets one
-    tile per split (4 KV heads of 64 tiles, one exact: 256 one-tile splits)."""
+    count fits ``slots`` resident workgroups, at most 64 entries per split.  Where every kept tile could
+    have a slot of its own, n_h is the head's tile count; the cuts still go by cost, so a head whose tiles
+    all cost the same gets one tile per split, and one of mixed costs a few two-tile runs beside as many
+    empty splits (4 KV heads of 64 tiles, kinds INT8, INT4, exact, INT8: the exact head 64 runs of one tile,
+    the others 60 or 61 runs, 3 or 4 of them of two tiles)."""
     costs = [entry_costs(m) for m in metas]
     heads = [c.sum(1) for c in costs]
     floors = [np.maximum((m["count"].numpy() + 63) // 64, 1) for m in metas]
