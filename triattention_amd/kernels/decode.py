@@ -425,12 +425,13 @@ class DecodeCache:
         the host and the device, and room for the task items that ``plan`` derives from them.  It depends on
         lengths, bands and the wave alone, so every prompt of one shape (each layer of a model, each new
         prompt) shares it; ragged batches of several stores compute their own.  Each stream has layouts of its
-        own: their device tensors go back to the stream they were made on."""
+        own: their device tensors go back to the stream they were made on.  A store under capture neither takes a
+        kept layout nor keeps its own: its uploads are refused there, whatever was stored before."""
         if self.wave is None:
             cus = self.module.device_cus() if hasattr(self.module, "device_cus") else \
                 torch.cuda.get_device_properties(st.device).multi_processor_count
             self.wave = cus * max(1, min(self.module.decode_occupancy(), SPLITS_PER_CU))
-        if len(st.groups) > 1:
+        if len(st.groups) > 1 or _capturing(st.device):
             return self._partition(st)
         g = st.groups[0]
         key = (g["meta"]["key"], g["batch"], st.maxn, st.grow_tiles, self.per, self.wave, _stream(st.device))
