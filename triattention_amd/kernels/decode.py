@@ -216,6 +216,7 @@ class _LayerStore:
         self.grow_tiles = 0
         self.tb = 0
         self.tail_clear = False  # the tails and the tail base are zero and no step has run on them
+        self.recorded = False  # some store was captured into a graph: every replay stores a prompt anew
         self.arrays["tail_base"] = torch.zeros(2, dtype=torch.int64, device=device)
 
     def _regrow(self, name, shape, fill, dtype, written=False):
@@ -382,6 +383,7 @@ class DecodeCache:
         if self.ragged and row0:
             a["count"][:row0].copy_(a["count0"][:row0])  # the earlier rows' tiles taken from their tails go
         st.rows += batch
+        st.recorded = st.recorded or _capturing(device)
         for k in seq:
             st.n[k] += batch * (seq[k] + room[k])
         st.groups.append(dict(prompt=prompt, batch=batch, hk=hk, tiles=tiles, meta=meta, exact=exact_kv, row0=row0,
@@ -595,7 +597,8 @@ class DecodeCache:
             hq = q.shape[1]
             if ("partials", hq) not in e:
                 e[("partials", hq)] = self._partials(e, q)
-            if tasks and "tasks" not in e:
+            # (a replay of a captured store brings other scales, which a table would not follow: such a cache gathers)
+            if tasks and "tasks" not in e and not e["store"].recorded:
                 self._build_tasks(e, q.device)
             e[key] = self._plan_decode(e, q, k, out, scale, e[("partials", hq)], e.get("tasks") if self.tasks else None)
         return e[key]
