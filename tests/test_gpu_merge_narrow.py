@@ -1,4 +1,4 @@
-"""GPU parity of the merge on narrow grids (eight waves per (sequence, q-head)).
+"""GPU parity of the merge on narrow grids (four or eight waves per (sequence, q-head)).
 
 Against the oracle's decode at the merge's own edges: split counts around one round (8 waves), the up-front loads
 (16, 32, 64 splits) and past them, and tails around the score rounds (64 tokens), the value rounds (32) and their
@@ -46,3 +46,51 @@ def test_narrow_merge_matches_the_oracle(module, tiles, per, tail):
                    bits(kt[-1].contiguous()), bits(vt[-1].contiguous()), tail - 1)
     err = np.abs(out[0, :, 0].cpu().numpy() - ref)
     assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, f"max {err.max():.3e} mean {err.mean():.3e}"
+
+
+@pytest.mark.parametrize("batch, tail, splits", [(1, 32, 64), (1, 33, 64), (1, 1, 65), (43, 1, 2), (43, 192, 3),
+                                                 (43, 193, 3)])
+def test_narrow_merge_around_its_choice_of_waves(module, batch, tail, splits):
+    """Either side of the tails and split counts at which the wave count changes, on grids of up to and of more than
+    a workgroup per CU: the merge of given partials and tail rows against the same sums in float64, each
+    (sequence, q-head) of its own; and a replay gives an eager step's bits."""
+    hq, hk, scale = 6, 2, 128 ** -0.5
+    assert (batch * hq <= module.device_cus()) == (batch == 1) and batch * hq < 2 * module.device_cus()
+    print(f"\n[merge] {batch} sequences, tail {tail}, {splits} splits", flush=True)
+    g = S.gen(9200 + tail)
+    prompt = 64 * splits
+    k, v = (S.outlier_tensor(g, 1, hk, prompt).expand(batch, -1, -1, -1).cuda() for _ in range(2))
+    cache = DecodeCache(module, max_tail=tail)
+    cache.per, cache.out_dtype = 1, torch.float32
+    Prefill(module, bands_fn_of(torch.tensor([[S.INF, S.INF]] * hq, dtype=torch.int32)), cache).store_only(0, k, v, hq)
+    e = cache.layers[0]
+    assert e["splits"] == splits
+    q, kt, vt = (torch.randn(batch, h, n, 128, generator=g).to(torch.bfloat16) for h, n in ((hq, 1), (hk, tail), (hk, tail)))
+    token = [x.contiguous().cuda() for x in (q, kt[:, :, -1:], vt[:, :, -1:])]
+    e["tail_k"][:, :, :tail - 1], e["tail_v"][:, :, :tail - 1] = kt[:, :, :-1].cuda(), vt[:, :, :-1].cuda()
+    cache.step.fill_(tail - 1)
+    cache.host_step = tail - 1
+    out = cache(0, *token, scale)
+    # float64: the partials are relative to the prompt's mean key, as the tail's scores are
+    pm, pl, po = (x.double().cpu() for x in e[("partials", hq)])
+    pm, pl, po = pm.view(batch, hq, splits), pl.view(batch, hq, splits), po.view(batch, hq, splits, 128)
+    mean = e["kstat"][:, :, 0].double().cpu()
+    vmean, vscale = e["vstat"][:, :, 0].double().cpu(), e["vstat"][:, :, 1].double().cpu()
+    rep = lambda x: x.repeat_interleave(hq // hk, 1)
+    s = (rep(kt.double() - mean[:, :, None]) * q.double()).sum(3) * (scale * np.log2(np.e))
+    m = torch.maximum(pm.amax(2), s.amax(2))[:, :, None]
+    wp, ws = torch.exp2(pm - m), torch.exp2(s - m)
+    prompt_o = (wp[..., None] * po).sum(2) * rep(vscale) + (wp * pl).sum(2)[..., None] * rep(vmean)
+    want = (prompt_o + (ws[..., None] * rep(vt.double())).sum(2)) / ((wp * pl).sum(2) + ws.sum(2))[..., None]
+    err = (out[:, :, 0].cpu().double() - want).abs()
+    assert float(err.max()) <= MAX_ABS and float(err.mean()) <= MEAN_ABS, f"max {err.max():.3e} mean {err.mean():.3e}"
+    graph = torch.cuda.CUDAGraph()
+    cache.begin_capture()
+    with torch.cuda.graph(graph):
+        again = cache(0, *token, scale)
+    cache.end_capture()
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, out)
+        again.zero_()

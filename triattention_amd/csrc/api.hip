@@ -533,6 +533,7 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
     int cus = 0;
     if (device_cus(&cus) != 0) return 1;
     mg.wide = (int64_t)batch * hq >= (int64_t)tri::SHORT_WIDE * cus ? 1 : 0;
+    mg.narrow_tail = tri::narrow_tail_of((int64_t)batch * hq, cus, splits);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (phase & 1) {
@@ -562,9 +563,8 @@ static int decode_impl(const void* q, int64_t q_sb, int64_t q_sh, const void* k8
   if (phase & 2) {
     // phase bit 4: the merge as one wave per (sequence, q-head), for short tails
     if (phase & 4) tri::decode_merge1_kernel<<<dim3(hq, batch), 64, 0, s>>>(mg);
-    // (a narrow grid's form does not depend on the tail: no choice on the device)
     else if (mg.wide) tri::decode_merge_kernel<<<dim3(hq, batch), 256, 0, s>>>(mg);
-    else tri::decode_merge_narrow_kernel<tri::MERGE_NARROW><<<dim3(hq, batch), 64 * tri::MERGE_NARROW, 0, s>>>(mg);
+    else tri::decode_merge_narrow_kernel<<<dim3(hq, batch), 64 * tri::MERGE_NARROW, 0, s>>>(mg);
   }
   return check_launch("decode");
 }

@@ -862,6 +862,7 @@ struct MergeArgs {
   int hq, hk, splits, max_tail;
   float sm_log2;
   int wide;  // the grid has at least SHORT_WIDE workgroups per CU (the one-wave form may pay)
+  int narrow_tail;  // on a narrower grid: the longest tail that four waves merge (narrow_tail_of)
 };
 
 // LSE merge of the split partials with the exact bf16 tail
@@ -875,11 +876,6 @@ struct MergeArgs {
 // of them.  Tail scores: 8 lanes per token (16 channels each); tail values: 16 lanes
 // per token (8 channels each).
 constexpr int MERGE_K = 2, MERGE_V = 4;
-// Waves per (sequence, q-head) on grids of fewer than SHORT_WIDE workgroups per CU, which leave SIMDs idle:
-// a long tail is bound by each wave's own scores and weights.  Kernel times at 4 / 8 / 16 waves: 256
-// workgroups, 700-token tails 16.9 / 11.7 / 12.0 us (19.9 with one round of K rows in flight and the splits past 16
-// one after another); 28 workgroups, 64 splits, 37-token tails 5.3 / 4.6 / 6.1 us (8.0).
-constexpr int MERGE_NARROW = 8;
 template <int NW>
 __device__ __forceinline__ void merge_waves(const MergeArgs& a) {
   constexpr int SG = 8 * NW, VG = 4 * NW;  // token groups of the score and value layouts
@@ -973,15 +969,21 @@ __device__ __forceinline__ void merge_waves(const MergeArgs& a) {
     if ((tid & 7) == 0 && t < tail) ts[t] = part * a.sm_log2;
   };
   score(kraw, sgrp);
-  // MERGE_K rounds of SG tokens in flight
-  for (int t0 = SG; t0 < tail; t0 += SG * MERGE_K) {
+  // MERGE_K rounds of SG tokens in flight, the last one alone where it is (a round past the tail would load and score
+  // the last row again: 896 workgroups, 8 splits, 41-token tails 8.7 us with it, 8.4 without)
+  int k0 = SG;
+  for (; k0 + SG * (MERGE_K - 1) < tail; k0 += SG * MERGE_K) {
     uint4 raw[MERGE_K][2];
 #pragma unroll
     for (int u = 0; u < MERGE_K; ++u)
-      krow(t0 + SG * u + sgrp, raw[u]);
+      krow(k0 + SG * u + sgrp, raw[u]);
 #pragma unroll
     for (int u = 0; u < MERGE_K; ++u)
-      score(raw[u], t0 + SG * u + sgrp);
+      score(raw[u], k0 + SG * u + sgrp);
+  }
+  for (; k0 < tail; k0 += SG) {
+    krow(k0 + sgrp, kraw);
+    score(kraw, k0 + sgrp);
   }
   float pm_own = pms;
   for (int s = 64 + lane; s < splits; s += 64) pm_own = fmaxf(pm_own, a.pm[pbase + s]);
@@ -1276,11 +1278,27 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(MergeArgs a) {
   }
 }
 
-// The merge of narrow grids (!a.wide), whose form does not depend on the tail: NW waves per (sequence, q-head).
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void decode_merge_narrow_kernel(MergeArgs a) {
-  merge_waves<NW>(a);
+// The merge of grids under SHORT_WIDE workgroups per CU, which leave SIMDs idle: eight waves per (sequence, q-head)
+// for a tail past a.narrow_tail tokens, where each wave's own scores and weights bound it (16 waves are no faster),
+// four up to there, where eight only start later and add up more partial sums.  The choice is made here as
+// decode_merge_kernel's is.
+constexpr int MERGE_NARROW = 8;
+__global__ __launch_bounds__(64 * MERGE_NARROW) void decode_merge_narrow_kernel(MergeArgs a) {
+  if (merge_tail(a) <= a.narrow_tail) {
+    if (threadIdx.x >= 256) return;  // (barriers wait for the surviving waves alone)
+    merge_waves<4>(a);
+  } else {
+    merge_waves<MERGE_NARROW>(a);
+  }
 }
+// The longest tail that four waves merge.  Up to a workgroup per CU: the 32 tokens that they score in one round.  More
+// workgroups share their CU's SIMDs: 192.  Past the 64 splits whose partials are loaded at once: none, as the others
+// go a round trip per wave of theirs.  Kernel times with four / eight waves, by tail tokens:
+//   56 workgroups, 54 splits: 1 5.0 / 5.3 us, 32 5.1 / 5.2, 33 5.5 / 5.3, 96 6.3 / 5.7, 700 16.0 / 10.5
+//   256 workgroups, 17 splits: 1 4.5 / 4.9, 32 4.6 / 5.0, 33 4.9 / 4.9, 96 5.8 / 5.4, 700 15.4 / 10.2
+//   384 workgroups, 11 splits: 1 5.0 / 6.0, 33 5.5 / 6.0, 96 6.3 / 6.6, 192 7.7 / 7.9, 256 8.8 / 8.6, 700 17.6 / 14.8
+//   56 workgroups, 137 splits: 1 7.4 / 6.5, 32 7.4 / 6.5, 700 17.6 / 11.7
+inline int narrow_tail_of(int64_t wgs, int cus, int splits) { return splits > 64 ? 0 : wgs <= cus ? 32 : 192; }
 
 // The one-wave form alone, whatever the tail (tri_decode_short_tail).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void decode_merge1_kernel(MergeArgs a) {
