@@ -87,6 +87,28 @@ def test_a_short_cache_is_cut_without_bisection(monkeypatch, tiles, batch, exact
     assert len(evaluations) <= (2 if batch * int(meta["count"].sum()) <= slots else 63)
 
 
+@pytest.mark.parametrize("per", [None, 3])
+@pytest.mark.parametrize("grow", [0, 128])
+def test_task_items_are_the_kept_splits_costliest_first(per, grow):
+    """Against every split's entries added up one by one, over stores of several lengths and batches."""
+    cache = DecodeCache(HostCacheModule(), max_tail=64, grow_tail=grow)
+    cache.ragged, cache.per = True, per
+    for prompt, batch in ((200, 2), (64, 1), (1500, 1), (130, 3)):
+        store(cache, 0, prompt, batch)
+    e = cache.layers[0]
+    costs = {}
+    for g in e["groups"]:
+        tile_costs, count = entry_costs(g["meta"]), g["meta"]["count"].tolist()
+        for s in range(g["row0"], g["row0"] + g["batch"]):
+            for h in range(2):
+                for i in range(e["splits"]):
+                    first, end = (i * e["per"], min((i + 1) * e["per"], count[h])) if e["bounds_host"] is None else \
+                        e["bounds_host"][s, h, i:i + 2].tolist()
+                    if first < end:  # (a growth split holds no kept tile yet: listed, at no cost)
+                        costs[(s * 2 + h) * e["splits"] + i] = tile_costs[h, first:min(end, count[h])].sum()
+    assert DecodeCache._task_items(e).tolist() == sorted(costs, key=lambda i: (-costs[i], i))
+
+
 def test_layouts_are_bounded():
     cache = DecodeCache(HostCacheModule(), max_tail=8)
     cache.LAYOUTS = 3

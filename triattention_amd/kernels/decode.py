@@ -118,10 +118,13 @@ def growth_kinds(bands, hk: int, exact_kv=()):
 def entry_costs(meta) -> np.ndarray:
     """Cost of each kept entry of one sequence [Hk, maxn] (float64, 0 past the count): the split
     kernel's measured time per tile of its kind (TILE_COST, plus K8_COST for INT8 K and V8_COST for
-    INT8 V; EXACT_COST for an exact head's tile)."""
+    INT8 V; EXACT_COST for an exact head's tile), kept with the metadata."""
+    if "costs" in meta:
+        return meta["costs"]
     exact = meta["exact"].numpy()[:, None]
     quant = TILE_COST + np.where(meta["is4"].numpy(), 0, K8_COST) + np.where(meta["vcode"].numpy() == I8, V8_COST, 0)
-    return np.where(meta["valid"].numpy(), np.where(exact, EXACT_COST, quant), 0).astype(np.float64)
+    meta["costs"] = np.where(meta["valid"].numpy(), np.where(exact, EXACT_COST, quant), 0).astype(np.float64)
+    return meta["costs"]
 
 
 def split_bounds(costs: np.ndarray, valid: np.ndarray, n: np.ndarray) -> np.ndarray:
@@ -736,27 +739,32 @@ class DecodeCache:
         (the split kernel's measured time per tile kind, entry_costs; ties by item): the kernel deals the
         listed splits to the XCDs round-robin in this order, so the long splits start first and every XCD
         gets its share of each cost."""
-        groups = e["groups"]
-        counts = np.concatenate([np.repeat(g["meta"]["count"].numpy()[None], g["batch"], 0) for g in groups])
-        per_group = [entry_costs(g["meta"]) for g in groups]
-        width = max(c.shape[1] for c in per_group)
-        costs = np.concatenate([np.repeat(np.pad(c, ((0, 0), (0, width - c.shape[1])))[None], g["batch"], 0)
-                                for c, g in zip(per_group, groups)])
-        cum = np.concatenate([np.zeros(costs.shape[:2] + (1,)), costs.cumsum(2)], 2)
-        if e["bounds_host"] is not None:
-            b = np.minimum(e["bounds_host"], counts[:, :, None])
-            nonempty = e["bounds_host"][:, :, 1:] > e["bounds_host"][:, :, :-1]
-        else:
-            first = np.arange(e["splits"])[None, None, :] * e["per"]
-            nonempty = first < counts[:, :, None]
-            b = np.minimum(np.concatenate([first, first[:, :, -1:] + e["per"]], 2), counts[:, :, None])
-        b = np.minimum(b, width)
-        split_cost = np.diff(np.take_along_axis(cum, b, 2), axis=2)
-        items = np.flatnonzero(nonempty.reshape(-1)).astype(np.int32)
+        # (the sequences of a group are cut alike: one of them stands for all)
+        items, costs, row = [], [], 0
+        for g in e["groups"]:
+            c, count = entry_costs(g["meta"]), g["meta"]["count"].numpy()[:, None]
+            cum = np.zeros((c.shape[0], c.shape[1] + 1))
+            np.cumsum(c, 1, out=cum[:, 1:])
+            if e["bounds_host"] is not None:
+                b = e["bounds_host"][row]
+                nonempty = b[:, 1:] > b[:, :-1]
+            else:
+                b = np.arange(e["splits"] + 1)[None, :] * e["per"]
+                nonempty = b[:, :-1] < count
+            ends = cum[np.arange(len(c))[:, None], np.minimum(b, count)]
+            cost = ends[:, 1:] - ends[:, :-1]
+            of_one = np.flatnonzero(nonempty)
+            first = np.arange(row, row + g["batch"]) * cost.size
+            items.append((first[:, None] + of_one).reshape(-1))
+            costs.append(np.tile(cost.reshape(-1)[of_one], g["batch"]))
+            row += g["batch"]
+        items = np.concatenate(items).astype(np.int32)
         if not items.size:
             return np.zeros(1, np.int32)
-        order = np.lexsort((items, -split_cost.reshape(-1)[items]))
-        return items[order]
+        costs = np.concatenate(costs)
+        # (whole numbers; numpy sorts 16-bit ones by radix)
+        below = costs.max() - costs
+        return items[np.argsort(below.astype(np.uint16) if below.max() < 1 << 16 else below, kind="stable")]
 
     def split_of(self, layer, b):
         """The split argument of the oracle's decode for sequence b of the layer: its bounds
