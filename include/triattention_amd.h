@@ -52,7 +52,7 @@ int tri_pack_v(const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int batc
                float* vstat, void* v16p, void* v8p, void* v4p, int32_t* v8sum, void* stream);
 
 /* No counterpart in the reference: tri_prepare_qk, tri_pack_v and (exact not NULL)
- * tri_pack_exact of one prompt in two launches (extension).  The arguments are
+ * tri_pack_exact of one prompt in two or three launches (extension).  The arguments are
  * theirs, with the same contracts; kpartial and vpartial are two scratch buffers
  * (tri_pack_v may otherwise reuse tri_prepare_qk's). */
 int tri_prepare(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb, int64_t k_sh,

@@ -1,4 +1,4 @@
-"""GPU parity of the two prepare launches (tri_prepare_qk, tri_pack_v, tri_pack_exact, tri_prepare).
+"""GPU parity of the prepare launches (tri_prepare_qk, tri_pack_v, tri_pack_exact, tri_prepare).
 
 Codes, scales, statistics and records are whole numbers or single correctly rounded operations: every
 array is held to the oracle bit for bit at every size, the expanded INT4 keys and the V8 sums to the records
@@ -66,7 +66,10 @@ def all_codes(q, k, v):
 
 @pytest.mark.parametrize("batch, hq, hk, t, layout", [
     (1, 6, 2, 1, "head"), (2, 3, 3, 64, "token"), (1, 4, 2, 65, "padded"), (1, 2, 1, 1025, "token"),
-    (2, 4, 4, 8193, "head"), (3, 8, 8, 3001, "padded")])
+    (2, 4, 4, 8193, "head"), (3, 8, 8, 3001, "padded"),
+    # either side of the sizes whose statistics a launch of their own completes: no call, the one call, the one call
+    # and pack_v, all three
+    (10, 2, 2, 380, "padded"), (10, 2, 2, 450, "token"), (14, 2, 2, 300, "head"), (40, 2, 2, 450, "token")])
 def test_prepare_matches_the_oracle_and_the_separate_calls(module, batch, hq, hk, t, layout):
     print(f"\n[prepare] batch={batch} hq={hq} hk={hk} t={t} {layout}", flush=True)
     g = S.gen(7000 + t)

@@ -104,7 +104,7 @@ static int device_cus(int* cus) {
 }
 
 // ---- prepare calls (tri_prepare_qk, tri_pack_v, tri_pack_exact, tri_prepare): argument checks of each part, and
-// the two launches that serve any combination of them
+// the two or three launches that serve any combination of them
 static int prepare_qk_args(tri::PrepareArgs& a, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k,
                            int64_t k_sb, int64_t k_sh, int64_t k_st, int batch, int hq, int hk, int t, void* q8,
                            float* qa, void* kp, float* ka, float* partial, float* kstat, void* q4, float* qa4,
@@ -214,11 +214,9 @@ static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) 
   const bool has_k = a.k8 != nullptr, has_v = a.vstat != nullptr;
   const int64_t stat = heads * (tri::STAT_BLOCKS / 4);
   const int64_t qwgs = a.q8 ? (int64_t)((a.t + 31) / 32) * a.hq * a.batch : 0;
-  // Tiles per record workgroup: one below 2 * RECORD_WGS workgroups per part (a short prompt then has a workgroup
-  // per tile), more beyond, so that the statistics each workgroup forms anew stay cheap beside its tiles.
-  a.per = (int)std::max<int64_t>(1, heads * tiles / tri::RECORD_WGS);
-  a.chunks = (int)((tiles + a.per - 1) / a.per);
-  const int64_t rec = heads * a.chunks, xwgs = a.exact ? heads * tiles : 0;
+  const int64_t rec = heads * tiles, xwgs = a.exact ? heads * tiles : 0;
+  const int kparts = has_k ? 1 : 0, vparts = has_v && !a.v_identity ? 1 : 0;  // (with statistics)
+  a.finalized = tri::finalize_pays(tiles, heads, kparts, vparts);
   const int64_t g1 = (has_k ? stat : 0) + (has_v && !a.v_identity ? stat : 0) + qwgs;
   const int64_t g2 = (has_k ? rec : 0) + (has_v ? rec : 0) + xwgs;
   if (g1 > INT32_MAX || g2 > INT32_MAX) return fail("%s: too many rows", what);
@@ -226,10 +224,15 @@ static int launch_prepare(tri::PrepareArgs& a, hipStream_t s, const char* what) 
   a.vstat_wgs = has_v && !a.v_identity ? (int)stat : 0;
   a.krec_wgs = has_k ? (int)rec : 0;
   a.vrec_wgs = has_v ? (int)rec : 0;
+  a.qblocks = tri::divisor((a.t + 31) / 32);
+  a.qheads = tri::divisor(a.hq);
+  a.kvheads = tri::divisor(a.hk);
+  a.ktiles = tri::divisor(tiles);
   for (int64_t w = 0; w < g1; w += PREPARE_GRID) {
     a.wg0 = (int)w;
     tri::prepare_stats_kernel<<<dim3((unsigned)std::min(PREPARE_GRID, g1 - w)), 256, 0, s>>>(a);
   }
+  if (a.finalized) tri::prepare_finalize_kernel<<<dim3((unsigned)((kparts + vparts) * heads)), 256, 0, s>>>(a);
   for (int64_t w = 0; w < g2; w += PREPARE_GRID) {
     a.wg0 = (int)w;
     tri::prepare_records_kernel<<<dim3((unsigned)std::min(PREPARE_GRID, g2 - w)), 256, 0, s>>>(a);

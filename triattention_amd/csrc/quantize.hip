@@ -8,12 +8,17 @@
 
 namespace tri {
 
-// Record workgroups per part (K, V): each takes max(1, tiles of all heads / RECORD_WGS) tiles, rounded down, so a
-// part of up to 2 * RECORD_WGS - 1 tiles has one per workgroup, and a longer one RECORD_WGS to 2 * RECORD_WGS - 1
-// workgroups (and at least one per head).  Fewer workgroups form the
-// statistics less often, more have more loads in flight (prepare_records_kernel at 256 / 512 / 1024 / 2048:
-// 4 x 8192 tokens, 4 KV heads, 46 / 41 / 46 / 52 us; 30,001 tokens, 8 KV heads, 76 / 72 / 66 / 80 us).
-constexpr int RECORD_WGS = 512;
+// n / d for n < 2^31 by a multiplication (a division of workgroup indexes costs a vector reciprocal and a dozen
+// dependent instructions before a workgroup's first load).
+struct Divisor {
+  uint32_t d, m, s;
+  __device__ __forceinline__ int quotient(int n) const { return (int)((__umulhi(m, (uint32_t)n) + (uint32_t)n) >> s); }
+};
+inline Divisor divisor(int64_t d) {
+  uint32_t s = 0;
+  while (((int64_t)1 << s) < d) ++s;
+  return Divisor{(uint32_t)d, (uint32_t)(((uint64_t)(((uint64_t)1 << s) - d) << 32) / d + 1), s};
+}
 
 // Arguments of one prepare call.  Parts that a call leaves out have a null source: q (the Q codes), k (K
 // statistics and records), v (V records; its statistics too unless v_identity), exact (KX / VX records).
@@ -38,16 +43,17 @@ struct PrepareArgs {
   const int32_t* exact;    // [hq]: 1 + record slot of the q-head's KV head, 0 if quantized
   int nx;
   uint8_t *kx, *vx;
-  // workgroups per part, tiles per record workgroup, and the launch's first workgroup (set by the host)
-  int kstat_wgs, vstat_wgs, krec_wgs, vrec_wgs, per, chunks, wg0;
+  // workgroups per part, and the launch's first workgroup (set by the host)
+  int kstat_wgs, vstat_wgs, krec_wgs, vrec_wgs, wg0;
+  Divisor qblocks, qheads, kvheads, ktiles;  // 32-row blocks of Q, q-heads, KV heads, tiles
+  int finalized;  // the statistics are complete (prepare_finalize_kernel): record workgroups read them
 };
 
 // Q codes: one 128-feature row per 8 lanes (16 features per lane, rotated with DPP lane moves by
 // rotate128_x16), 32 rows per 256-thread workgroup.  common_device.cuh:1-28 (quantize_q_kernel).
 __device__ __forceinline__ void quantize_q_rows(const PrepareArgs& a, int wg) {
-  const int blocks = (a.t + 31) / 32;
-  const int sub = threadIdx.x & 7, row = (wg % blocks) * 32 + (threadIdx.x >> 3);
-  const int h = (wg / blocks) % a.hq, b = wg / (blocks * a.hq);
+  const int hw = a.qblocks.quotient(wg), b = a.qheads.quotient(hw), h = hw - b * a.hq;
+  const int sub = threadIdx.x & 7, row = (wg - hw * (int)a.qblocks.d) * 32 + (threadIdx.x >> 3);
   if (row >= a.t) return;  // whole 8-lane groups leave together
   const uint16_t* src = a.q + b * a.qsb + h * a.qsh + (int64_t)row * a.qst + sub * 16;
   float x[16];
@@ -135,15 +141,16 @@ __device__ __forceinline__ void stat_block(const uint16_t* __restrict__ src, int
 // nothing but the inputs.  The statistics are latency-bound (64 serial sums per head and channel pair, one
 // wave each) and come first in the grid; the Q codes are HBM-bound and fill the rest of the chip meanwhile
 // (64 VGPRs at most, so that eight waves per SIMD keep their loads in flight).  Against a launch each
-// (Q codes, K partials, V partials): 4 x 8192 tokens, Hq 28 / Hk 4, 111 -> 105 us (4.6 TB/s, a plain copy
-// reaches 4.85); 30,001 tokens, Hq 32 / Hk 8, 163 -> 109 us; 1,024 tokens, Hq 24 / Hk 8, 14 -> 7.8 us.
+// (Q codes, K partials, V partials): 4 x 8192 tokens, Hq 28 / Hk 4, 108 -> 98 us (4.9 TB/s, as a plain copy;
+// 108 with the indexes of a workgroup by division); 30,001 tokens, Hq 32 / Hk 8, 160 -> 108 us (117); 1,024 tokens,
+// Hq 24 / Hk 8, 10.8 (and two launches) -> 7.2 us.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void prepare_stats_kernel(PrepareArgs a) {
   int wg = a.wg0 + blockIdx.x;
   if (wg < a.kstat_wgs + a.vstat_wgs) {
     const bool isv = wg >= a.kstat_wgs;
     if (isv) wg -= a.kstat_wgs;
     const int hb = wg / (STAT_BLOCKS / 4), blk = (wg % (STAT_BLOCKS / 4)) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int hd = hb % a.hk, b = hb / a.hk;
+    const int b = a.kvheads.quotient(hb), hd = hb - b * a.hk;
     const uint16_t* src = isv ? a.v + b * a.vsb + hd * a.vsh : a.k + b * a.ksb + hd * a.ksh;
     stat_block(src, isv ? a.vst : a.kst, a.t, blk, (isv ? a.vpart : a.kpart) + (int64_t)hb * STAT_BLOCKS * 3 * D);
     return;
@@ -152,8 +159,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
 }
 
 // Statistics of one head from its block partials: mean = (sum of block sums in block order) / T, scale =
-// range/127 (1 if 0), inv = 1/scale.  common_device.cuh:44-56 (finalize_kernel).  Every record workgroup
-// forms them again (96 KiB of partials, L2-resident) instead of waiting for a launch that does nothing
+// range/127 (1 if 0), inv = 1/scale.  common_device.cuh:44-56 (finalize_kernel).  In a call of few heads every record
+// workgroup forms them again (L2-resident partials) instead of waiting for a launch that does nothing
 // else.  256 threads: one half adds the channel's block sums, the other takes its extremes; mean and
 // inv (LDS, 128 each) are complete after the call's barrier.  stat (when not null) receives all three.
 // `range`: whether scale and inv are needed (a K record needs the mean alone).
@@ -428,12 +435,35 @@ __device__ __forceinline__ void pack_exact_tile(const uint16_t* ksrc, int64_t ks
   }
 }
 
-// Second launch of a prepare call: the K records, the V records and the exact heads' KX / VX records.  A K
-// or V workgroup forms its head's statistics from the block partials, then takes a.per consecutive tiles;
-// the first one of a head writes the statistics out.  HBM-bound for long prompts, latency-bound for short
-// ones: a tile's rows are loaded before the statistics, and the next tile's while one is worked on.
-// Against launches of their own for each head's statistics (K, V), the K, V and KX / VX records: 4 x 8192
-// tokens, 4 KV heads (one exact), 54 -> 41 us; 1,024 tokens, 8 KV heads, 20 -> 9 us.
+// The statistics of every (part, head), one workgroup each, for the calls whose record workgroups read them.
+__global__ __launch_bounds__(256) void prepare_finalize_kernel(PrepareArgs a) {
+  __shared__ float mean[D], inv[D], hi[D], lo[D];
+  const int heads = a.hk * a.batch, hb = blockIdx.x % heads;
+  const bool isv = a.kstat_wgs == 0 || (int)blockIdx.x >= heads;
+  head_stats((isv ? a.vpart : a.kpart) + (int64_t)hb * STAT_BLOCKS * 3 * D, a.t, true, mean, inv, hi, lo,
+             (isv ? a.vstat : a.kstat) + (int64_t)hb * 3 * D);
+}
+
+// Whether a finalize launch pays, for `heads` (sequence, KV head) pairs of `tiles` tiles and the parts (0 or 1 each)
+// that have statistics.  It costs a launch (~1.5 us); without it every record workgroup reads its head's partials (32
+// KiB of K's, 96 of V's), which is free while they are few, and not once many heads' partials pass through every
+// XCD's 4 MiB L2.  Calls without / with it, K, V (K and V): 4 heads x 64 tiles 25.7 / 27.4 us, 8 x 64 29.7 / 30.1, 32 x 8
+// 24.2 / 22.5, 80 x 8 45.2 / 39.3, 8 x 219 77.2 / 73.2, 32 x 469 680 / 609; K alone, 32 x 24 32.1 / 33.3, 80 x 8 33.5 /
+// 32.0, 32 x 64 67.3 / 65.5; V alone, 16 x 16 13.4 / 13.4, 32 x 8 16.3 / 14.0, 80 x 2 17.5 / 16.7.
+inline bool finalize_pays(int64_t tiles, int64_t heads, int kparts, int vparts) {
+  const int64_t partials = heads * (32 * kparts + 96 * vparts), work = heads * tiles;
+  return partials > 0 && tiles > 1 && ((partials >= 2560 && work >= (vparts ? 128 : 512)) || work >= 1280);
+}
+
+// Last launch of a prepare call: the K records, the V records and the exact heads' KX / VX records, one workgroup per
+// tile.  A K or V workgroup takes its head's statistics from prepare_finalize_kernel or forms them from the block
+// partials (finalize_pays); then the one of a head's first tile writes them out.  HBM-bound for long prompts,
+// latency-bound for short ones: a tile's rows are loaded before the statistics.  Against launches of their own for
+// each head's statistics (K, V) and the K and V records: 1,024 tokens, 8 KV heads, 14.5 (and three launches) -> 7.2 us;
+// with the finalize launch, 30,001 tokens, 8 KV heads, 71 -> 60 us, 4 x 8192 tokens, 4 KV heads, 47 -> 40 us, 4 x 30,000
+// tokens, 8 KV heads, 263 -> 219 us.  (With up to 1,088 workgroups of several tiles each, the next one's rows loaded
+// ahead, and the statistics formed in each: 76, 41 and 276 us; two tiles per workgroup after the finalize launch are
+// 4% slower than one.)
 __global__ __launch_bounds__(256) void prepare_records_kernel(PrepareArgs a) {
   // one staging buffer for the three parts: V' of a tile (fp32), K codes (one byte each, INT8 and INT4), or
   // the exact heads' bf16 V
@@ -443,62 +473,60 @@ __global__ __launch_bounds__(256) void prepare_records_kernel(PrepareArgs a) {
   static_assert(sizeof(stage) >= 2 * BN * D && sizeof(stage) >= BN * EXACT_VP * 2, "staging");
   const int tiles = (a.t + BN - 1) / BN;
   int wg = a.wg0 + blockIdx.x;
-  if (wg < a.krec_wgs) {
-    const int hb = wg / a.chunks, j0 = (wg % a.chunks) * a.per, j1 = min(tiles, j0 + a.per);
-    const int hd = hb % a.hk, b = hb / a.hk;
-    const uint16_t* src = a.k + b * a.ksb + hd * a.ksh;
-    KRaw cur, nxt;
-    load_k_tile(cur, src + (int64_t)j0 * BN * a.kst, a.kst, a.t - j0 * BN);
-    head_stats(a.kpart + (int64_t)hb * STAT_BLOCKS * 3 * D, a.t, j0 == 0, mean, inv, hi, lo,
-               j0 == 0 ? a.kstat + (int64_t)hb * 3 * D : nullptr);
-    auto* c8 = reinterpret_cast<uint8_t (*)[D]>(&stage[0][0]);
-    for (int j = j0; j < j1; ++j) {
-      const int64_t rec = (int64_t)hb * tiles + j;
-      if (j + 1 < j1) load_k_tile(nxt, src + (int64_t)(j + 1) * BN * a.kst, a.kst, a.t - (j + 1) * BN);
-      if (j > j0) __syncthreads();  // (the previous tile's codes are read)
-      quantize_k_tile(cur, a.t - j * BN, mean, a.k8 + rec * K8_BYTES, a.ka + rec * 4,
+  if (wg < a.krec_wgs + a.vrec_wgs) {
+    const bool isv = wg >= a.krec_wgs;
+    if (isv) wg -= a.krec_wgs;
+    const int hb = a.ktiles.quotient(wg), j = wg - hb * tiles, b = a.kvheads.quotient(hb), hd = hb - b * a.hk;
+    const int rows = a.t - j * BN;
+    const int64_t rec = (int64_t)hb * tiles + j;
+    // the head's statistics into LDS; where they come from the partials, the workgroup of tile 0 writes them out
+    auto stats = [&](const float* part, float* stat, bool range) {
+      part += (int64_t)hb * STAT_BLOCKS * 3 * D;
+      stat += (int64_t)hb * 3 * D;
+      if (a.finalized) {
+        if (threadIdx.x < D) mean[threadIdx.x] = stat[threadIdx.x];
+        else inv[threadIdx.x - D] = stat[D + threadIdx.x];  // (threads D to 2 D - 1: stat[2 D + channel])
+        __syncthreads();
+      } else {
+        head_stats(part, a.t, range || j == 0, mean, inv, hi, lo, j == 0 ? stat : nullptr);
+      }
+    };
+    if (!isv) {
+      KRaw raw;
+      load_k_tile(raw, a.k + b * a.ksb + hd * a.ksh + (int64_t)j * BN * a.kst, a.kst, rows);
+      stats(a.kpart, a.kstat, false);
+      auto* c8 = reinterpret_cast<uint8_t (*)[D]>(&stage[0][0]);
+      quantize_k_tile(raw, rows, mean, a.k8 + rec * K8_BYTES, a.ka + rec * 4,
                       a.k4 != nullptr ? a.k4 + rec * K4_BYTES : nullptr, a.k4 != nullptr ? a.ka4 + rec * 4 : nullptr, c8,
                       c8 + BN, a.k4x != nullptr ? a.k4x + rec * K8_BYTES : nullptr);
-      cur = nxt;
+      return;
     }
-    return;
-  }
-  wg -= a.krec_wgs;
-  if (wg < a.vrec_wgs) {
-    const int hb = wg / a.chunks, j0 = (wg % a.chunks) * a.per, j1 = min(tiles, j0 + a.per);
-    const int hd = hb % a.hk, b = hb / a.hk;
-    const uint16_t* src = a.v + b * a.vsb + hd * a.vsh;
-    VRaw cur, nxt;
-    load_v_tile(cur, src + (int64_t)j0 * BN * a.vst, a.vst, a.t - j0 * BN);
-    float* stat = j0 == 0 ? a.vstat + (int64_t)hb * 3 * D : nullptr;
+    VRaw raw;
+    load_v_tile(raw, a.v + b * a.vsb + hd * a.vsh + (int64_t)j * BN * a.vst, a.vst, rows);
     if (!a.v_identity) {
-      head_stats(a.vpart + (int64_t)hb * STAT_BLOCKS * 3 * D, a.t, true, mean, inv, hi, lo, stat);
+      stats(a.vpart, a.vstat, true);
     } else {
       if (threadIdx.x < D) {
         mean[threadIdx.x] = 0.f;
         inv[threadIdx.x] = 1.f;
-        if (stat != nullptr) {
-          stat[threadIdx.x] = 0.f;
-          stat[D + threadIdx.x] = 1.f;
-          stat[2 * D + threadIdx.x] = 1.f;
+        if (j == 0) {
+          float* stat = a.vstat + (int64_t)hb * 3 * D + threadIdx.x;
+          stat[0] = 0.f;
+          stat[D] = 1.f;
+          stat[2 * D] = 1.f;
         }
       }
       __syncthreads();
     }
-    for (int j = j0; j < j1; ++j) {
-      const int64_t rec = (int64_t)hb * tiles + j;
-      if (j + 1 < j1) load_v_tile(nxt, src + (int64_t)(j + 1) * BN * a.vst, a.vst, a.t - (j + 1) * BN);
-      if (j > j0) __syncthreads();  // (the previous tile's values and sums are read)
-      pack_v_tile(cur, a.t - j * BN, mean, inv, a.v16 != nullptr ? a.v16 + rec * V16_BYTES : nullptr,
-                  a.v8 != nullptr ? a.v8 + rec * V8_BYTES : nullptr, a.v4 != nullptr ? a.v4 + rec * V4_BYTES : nullptr,
-                  stage, a.v8s != nullptr ? a.v8s + rec * D : nullptr, vsum);
-      cur = nxt;
-    }
+    pack_v_tile(raw, rows, mean, inv, a.v16 != nullptr ? a.v16 + rec * V16_BYTES : nullptr,
+                a.v8 != nullptr ? a.v8 + rec * V8_BYTES : nullptr, a.v4 != nullptr ? a.v4 + rec * V4_BYTES : nullptr,
+                stage, a.v8s != nullptr ? a.v8s + rec * D : nullptr, vsum);
     return;
   }
+  wg -= a.krec_wgs;
   wg -= a.vrec_wgs;
   // exact heads: workgroup (KV head, tile) of sequence b; other heads leave
-  const int tile = wg % tiles, kh = (wg / tiles) % a.hk, b = wg / (tiles * a.hk);
+  const int hb = a.ktiles.quotient(wg), tile = wg - hb * tiles, b = a.kvheads.quotient(hb), kh = hb - b * a.hk;
   const int slot = a.exact[kh * (a.hq / a.hk)] - 1;
   if (slot < 0 || slot >= a.nx) return;
   const int64_t rec = ((int64_t)b * a.nx + slot) * tiles + tile;

@@ -218,7 +218,7 @@ class Module:
     # ----------------------------------------------------------------- prepare
     def prepare(self, q, k, v, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x, vpartial, vstat, v16p, v8p,
                 v4p, v8sum, exact=None, nx=0, kx=None, vx=None):
-        """``prepare_qk``, ``pack_v`` and (with ``exact``) ``pack_exact`` of one prompt in two launches
+        """``prepare_qk``, ``pack_v`` and (with ``exact``) ``pack_exact`` of one prompt in two or three launches
         (extension): the same buffers with the same contents, K's and V's statistics partials in
         scratch buffers of their own."""
         b, hq, hk, t = self._check_qk(q, k, q8, qa, kp, ka, kpartial, kstat, q4, qa4, k4p, ka4, k4x)
