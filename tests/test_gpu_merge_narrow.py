@@ -94,3 +94,29 @@ def test_narrow_merge_around_its_choice_of_waves(module, batch, tail, splits):
         torch.cuda.synchronize()
         assert torch.equal(again, out)
         again.zero_()
+
+
+@pytest.mark.parametrize("tail, tiles", [(17, 1), (20, 10), (32, 23)])
+def test_a_short_tail_merges_alike_on_narrow_and_wide_grids(module, tail, tiles):
+    """One sequence alone and among copies of itself that make the grid wide: the same bits (four waves either way, the
+    splits summed in one order)."""
+    hq, hk, scale, per = 6, 2, 128 ** -0.5, 1
+    copies = -(-2 * module.device_cus() // hq)
+    print(f"\n[merge] tail {tail}, {tiles} tiles, alone and {copies} times", flush=True)
+    g = S.gen(9400 + tail)
+    k, v = S.outlier_tensor(g, 1, hk, 64 * tiles).cuda(), S.outlier_tensor(g, 1, hk, 64 * tiles).cuda()
+    kt, vt = (torch.randn(1, hk, tail, 128, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    q = torch.randn(1, hq, 1, 128, generator=g).to(torch.bfloat16).cuda()
+    outs = []
+    for batch in (1, copies):
+        many = lambda x: x.expand(batch, -1, -1, -1).contiguous()
+        cache = DecodeCache(module, max_tail=tail)
+        cache.per, cache.out_dtype = per, torch.float32
+        bands = torch.tensor([[S.INF, S.INF]] * 3 + [[1, S.INF]] * 3, dtype=torch.int32)
+        Prefill(module, bands_fn_of(bands), cache).store_only(0, many(k), many(v), hq)
+        e = cache.layers[0]
+        e["tail_k"][:, :, :tail - 1], e["tail_v"][:, :, :tail - 1] = kt[:, :, :-1], vt[:, :, :-1]
+        cache.step.fill_(tail - 1)
+        cache.host_step = tail - 1
+        outs.append(cache(0, many(q), many(kt[:, :, -1:]), many(vt[:, :, -1:]), scale))
+    assert torch.equal(outs[1], outs[0].expand(copies, -1, -1, -1))
